@@ -14,6 +14,9 @@ int g4_num_cus();
 // device address of the allocation-free attention's scratch on `device`
 // (current), resolved once per device; called by g4_init
 int g4_attn_scratch_setup(int device);
+// g4_mm_batch of Q6_K / bf16 weights on fp32 activations (arguments checked:
+// n a multiple of 256, x and w 16-byte aligned)
+int g4_mm_batch_f32(float* o, const float* x, const void* w, int n, int d, int m, int type);
 // last pass of an argmax over np per-workgroup keys (argmax_key order):
 // the index to *out / *dtok (each optional), *dpos advanced if given
 int g4_argmax_final(const void* part, int np, int* out, int* dtok, int* dpos);

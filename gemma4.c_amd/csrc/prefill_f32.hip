@@ -1,0 +1,520 @@
+// prefill_f32.hip -- Y[m x d] = X[m x n] . W[d x n]^T for fp32 activations
+// and Q6_K or bf16 weights on the 16-bit matrix cores (g4_mm_batch; the
+// reference's mm_quant_rows and mm_bf16 once per token,
+// gemma4-4b/cpu-blas/main.c:1539-1556, 1529-1537).
+//
+// Products.  bf16: an fp32 activation is the exact sum of three bf16 terms
+// (8 + 8 + 8 significant bits, by truncation), so three
+// v_mfma_f32_16x16x32_bf16 give the fp32 path's products exactly.  Q6_K: over
+// 64 elements of a token the activations are scaled by the power of two that
+// brings the largest into [2^14, 2^15) and split into two fp16 terms (within
+// 2^-22 of each element), the integer weight sc * (q - 32) exactly into
+// Wh + Wl as in mm_batch_q6s_kernel; three v_mfma_f32_16x16x32_f16, then one
+// multiplication by the token's scale and one FMA with the block's d.
+// Outputs that are not finite are computed again by plain fp32 dots, so
+// infinities and NaN in either operand behave as in the fp32 product.
+//
+// Work split.  The four waves of a workgroup share one output tile and split
+// K: wave w takes the Q6_K blocks b = w (mod 4), or of every 256 bf16
+// elements those from 64 w, and the four partial tiles are added through LDS
+// at the end, (a0 + a1) + (a2 + a3).  A wave thus loads each operand once,
+// straight into the registers it feeds the matrix cores from (no staging, no
+// barrier in the loop), and splits each activation and decodes each weight
+// once per workgroup.  The order of a token's sums depends on n alone, so
+// every tile shape gives the same bits.
+#include "g4_device.h"
+#include "g4_internal.h"
+#include "g4_tile.h"
+
+namespace g4 {
+namespace {
+
+typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
+
+// the sum over the four waves' partial tiles and the store.  Weights are the
+// A operand: lane (g, i) holds weight rows 4g + v of 16-row group rt and token
+// i of 16-token group nt.  T: 16x16 tiles per wave; red_tiles(T) of them
+// pass through LDS at a time.
+constexpr int red_tiles(int t) { return t < 10 ? t : 10; }
+
+template <int NT, int RT, class Slow>
+__device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, float* __restrict__ out, int row0, int tok0,
+                                             int d, int m, bool vec, Slow slow) {
+    constexpr int T = NT * RT, R = red_tiles(T);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int t0 = 0; t0 < T; t0 += R) {
+        if (t0) __syncthreads();
+#pragma unroll
+        for (int t = t0; t < t0 + R; t++)
+            if (t < T) red[(wave * R + (t - t0)) * 64 + lane] = acc[t / NT][t % NT];
+        __syncthreads();
+#pragma unroll
+        for (int t = t0; t < t0 + R; t++) {
+            if (t >= T || (t & 3) != wave) continue;
+            const f4_t* r = red + (t - t0) * 64 + lane;
+            const f4_t a = r[0], b = r[R * 64], c = r[2 * R * 64], e = r[3 * R * 64];
+            const int row = row0 + 16 * (t / NT) + 4 * g, tok = tok0 + 16 * (t % NT) + i;
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] = (a[k] + b[k]) + (c[k] + e[k]);
+                if (tok < m && row + k < d && !(fabsf(v[k]) <= 3.402823466e38f)) v[k] = slow(tok, row + k);
+            }
+            if (tok >= m) continue;
+            float* o = out + (size_t)tok * d + row;
+            if (vec && row + 3 < d) {
+                *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (row + k < d) o[k] = v[k];
+            }
+        }
+    }
+}
+
+// ---- bf16 weights ---------------------------------------------------------
+template <int NT, int RT>
+__global__ __launch_bounds__(256) void mm_batch_bf16_kernel(const uint16_t* __restrict__ w, const float* __restrict__ x,
+                                                            float* __restrict__ out, int n, int d, int m, int vec) {
+    __shared__ f4_t red[4 * red_tiles(NT * RT) * 64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    int bx, by;
+    xcd_tile((m + 16 * NT - 1) / (16 * NT), bx, by);
+    const int row0 = bx * 16 * RT, tok0 = by * 16 * NT;
+    const int nb = n >> 8;
+    // of the wave's 64 elements of a block, lane group g takes 16 g .. + 15 and
+    // step s of the two 16 g + 8 s .. + 7
+    const float* px[NT];
+    const uint16_t* pw[RT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) px[nt] = x + (size_t)min(tok0 + 16 * nt + i, m - 1) * n + 64 * wave + 8 * g;
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) pw[rt] = w + (size_t)min(row0 + 16 * rt + i, d - 1) * n + 64 * wave + 8 * g;
+
+    struct Ops {
+        uint4 x[NT][4];
+        uint4 w[RT][2];
+    };
+    auto load = [&](int b, Ops& r) {
+        const size_t o = (size_t)b * 256;
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) r.x[nt][k] = reinterpret_cast<const uint4*>(px[nt] + o + 32 * (k >> 1))[k & 1];
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) r.w[rt][k] = *reinterpret_cast<const uint4*>(pw[rt] + o + 32 * k);
+    };
+    f4_t acc[RT][NT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) acc[rt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const Ops& r) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            b8_t xt[3][NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                uint32_t f[8] = {r.x[nt][2 * s].x,     r.x[nt][2 * s].y,     r.x[nt][2 * s].z,     r.x[nt][2 * s].w,
+                                 r.x[nt][2 * s + 1].x, r.x[nt][2 * s + 1].y, r.x[nt][2 * s + 1].z, r.x[nt][2 * s + 1].w};
+#pragma unroll
+                for (int t = 0; t < 3; t++) {
+                    uint32_t p[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) p[k] = __builtin_amdgcn_perm(f[2 * k + 1], f[2 * k], 0x07060302u);
+                    xt[t][nt] = __builtin_bit_cast(b8_t, make_uint4(p[0], p[1], p[2], p[3]));
+                    if (t == 2) break;
+#pragma unroll
+                    for (int k = 0; k < 8; k++)   // exact: the bits below the term's
+                        f[k] = __float_as_uint(__uint_as_float(f[k]) - __uint_as_float(f[k] & 0xffff0000u));
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                const b8_t a = __builtin_bit_cast(b8_t, r.w[rt][s]);
+#pragma unroll
+                for (int t = 2; t >= 0; t--)
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++)
+                        acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, xt[t][nt], acc[rt][nt], 0, 0, 0);
+            }
+        }
+    };
+    // the next block's operands load while the current one's are multiplied
+    // (past the end the last block again: no branch around the loads)
+    Ops r0, r1;
+    load(0, r0);
+    int b = 0;
+    for (; b + 1 < nb; b += 2) {
+        load(b + 1, r1);
+        compute(r0);
+        load(min(b + 2, nb - 1), r0);
+        compute(r1);
+    }
+    if (b < nb) compute(r0);
+
+    reduce_store<NT, RT>(acc, red, out, row0, tok0, d, m, vec, [&](int tok, int row) {
+        float sum = 0.0f;
+        for (int k = 0; k < n; k++)
+            sum = __builtin_fmaf(__uint_as_float((uint32_t)w[(size_t)row * n + k] << 16), x[(size_t)tok * n + k], sum);
+        return sum;
+    });
+}
+
+// ---- bf16 weights on the fp32 matrix cores -----------------------------------
+// g4_mm_batch_bf16_f32: fp32 products and one running fp32 sum per output
+// (v_mfma_f32_16x16x4_f32).  A prompt's per-layer-embedding projection stays
+// on it (0.27 ms of a 511-token E4B prompt against 0.16 ms): its rows end up in
+// 8-bit codes, where a sum in another order moves some code by one and the
+// model carries that on, so a prompt would no longer give the bits, nor always
+// the tokens, it gave before.
+//
+// The 16 tokens of a tile are the A rows, 16 weight rows the B columns, so a
+// lane's results are one weight row of four tokens.  Lane group g supplies K
+// index g of every 16x16x4 step; over one 256-long block it walks elements
+// 64 g .. 64 g + 63 of its row.  The activations of the workgroup's tokens are
+// staged per block in LDS in natural order (260 floats per token:
+// conflict-free 16-byte reads).
+constexpr int kF32XS = 260;
+
+template <int RW, int NT>
+__global__ __launch_bounds__(64 * RW) void mm_batch_f32_kernel(const uint16_t* __restrict__ w,
+                                                               const float* __restrict__ x, float* __restrict__ out,
+                                                               int n, int d, int m) {
+    constexpr int NTHR = 64 * RW;
+    constexpr int TOK = 16 * NT;
+    constexpr int XV = TOK * 64 / NTHR;             // float4 of activations per thread and block
+    static_assert(XV * NTHR == TOK * 64, "token tile must divide among the threads");
+    __shared__ __align__(16) float sx[TOK * kF32XS];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.x * (16 * RW) + wave * 16;
+    const int tok0 = blockIdx.y * TOK;
+    const int nb = n >> 8;
+    const size_t rj = (size_t)min(row0 + i, d - 1);  // this lane's weight row
+
+    struct WRaw {
+        uint4 v[8];     // 64 values
+    };
+    auto load_w = [&](int b, WRaw& r) {
+        const uint4* p = reinterpret_cast<const uint4*>(w + rj * n + (size_t)b * 256 + 64 * g);
+#pragma unroll
+        for (int k = 0; k < 8; k++) r.v[k] = p[k];
+    };
+    struct XRaw {
+        f4_t v[XV];
+    };
+    // unit u = tid + j * NTHR: token u >> 6, float4 u & 63 of the block
+    auto load_x = [&](int b, XRaw& r) {
+#pragma unroll
+        for (int j = 0; j < XV; j++) {
+            const int u = tid + j * NTHR;
+            const int t = min(tok0 + (u >> 6), m - 1);
+            r.v[j] = reinterpret_cast<const f4_t*>(x + (size_t)t * n + (size_t)b * 256)[u & 63];
+        }
+    };
+    auto stage = [&](const XRaw& r) {
+#pragma unroll
+        for (int j = 0; j < XV; j++) {
+            const int u = tid + j * NTHR;
+            *reinterpret_cast<f4_t*>(sx + (u >> 6) * kF32XS + 4 * (u & 63)) = r.v[j];
+        }
+    };
+
+    f4_t acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[t] = f4_t{0.f, 0.f, 0.f, 0.f};
+
+    WRaw wn;
+    XRaw xn;
+    load_w(0, wn);
+    load_x(0, xn);
+    for (int b = 0; b < nb; b++) {
+        lds_barrier();   // the previous block's LDS reads are done
+        stage(xn);
+        const WRaw wc = wn;
+        // the next block (the last one again at the end: an unconditional
+        // load keeps the prefetch registers out of scratch memory)
+        const int bn = min(b + 1, nb - 1);
+        load_w(bn, wn);
+        load_x(bn, xn);
+        lds_barrier();
+
+        const float* xa = sx + i * kF32XS;
+#pragma unroll
+        for (int t4 = 0; t4 < 16; t4++) {
+            const uint32_t lo = t4 & 1 ? wc.v[t4 >> 1].z : wc.v[t4 >> 1].x;
+            const uint32_t hi = t4 & 1 ? wc.v[t4 >> 1].w : wc.v[t4 >> 1].y;
+            const float wv[4] = {__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u),
+                                 __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)};
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const float4 a = *reinterpret_cast<const float4*>(xa + 16 * t * kF32XS + 64 * g + 4 * t4);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, wv[0], acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, wv[1], acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, wv[2], acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, wv[3], acc[t], 0, 0, 0);
+            }
+        }
+    }
+    // lane (g, i) holds tokens 4g + v of each tile, weight row row0 + i
+    const int row = row0 + i;
+    if (row < d) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int tok = tok0 + 16 * t + 4 * g + v;
+                if (tok < m) out[(size_t)tok * d + row] = acc[t][v];
+            }
+    }
+}
+
+// ---- Q6_K weights -----------------------------------------------------------
+template <int NT, int RT>
+__global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
+                                                          float* __restrict__ out, int n, int d, int m, int vec) {
+    __shared__ f4_t red[4 * red_tiles(NT * RT) * 64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 15, g = lane >> 4, h = g >> 1, s = g & 1;
+    int bx, by;
+    xcd_tile((m + 16 * NT - 1) / (16 * NT), bx, by);
+    const int row0 = bx * 16 * RT, tok0 = by * 16 * NT;
+    const int nb = n >> 8;
+    const size_t nblk = (size_t)d * nb;
+    const Q6KPlanes P = q6k_planes(nblk);
+
+    // lane group g's elements of a block: 128 h + 32 k + 16 s + 8 half + t, in
+    // step c = 2 k + half (layout.hip); group k of two steps is 16 in a row
+    const float* px[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) px[nt] = x + (size_t)min(tok0 + 16 * nt + i, m - 1) * n + 128 * h + 16 * s;
+    size_t rB[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) rB[rt] = (size_t)min(row0 + 16 * rt + i, d - 1) * nb;
+    const uint8_t* wql = w + P.ql + 32 * g;
+    const uint8_t* wqh = w + P.qh + 16 * g;
+    const uint8_t* wsc = w + P.sc + 8 * h;
+    const uint8_t* wd = w + P.d;
+
+    struct WRaw {
+        uint4 ql[RT][2];
+        uint4 qh[RT];
+        uint2 sc[RT];
+        uint32_t dh[RT];
+    };
+    struct XRaw {
+        f4_t v[NT][4];
+    };
+    auto load_w = [&](int b, WRaw& r) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            const size_t blk = rB[rt] + b;
+            r.ql[rt][0] = reinterpret_cast<const uint4*>(wql + blk * 128)[0];
+            r.ql[rt][1] = reinterpret_cast<const uint4*>(wql + blk * 128)[1];
+            r.qh[rt] = *reinterpret_cast<const uint4*>(wqh + blk * 64);
+            r.sc[rt] = *reinterpret_cast<const uint2*>(wsc + blk * 16);
+            r.dh[rt] = *reinterpret_cast<const uint16_t*>(wd + blk * 2);
+        }
+    };
+    auto load_x = [&](int b, int k, XRaw& r) {
+        const size_t o = (size_t)b * 256 + 32 * k;
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) r.v[nt][q] = reinterpret_cast<const f4_t*>(px[nt] + o)[q];
+    };
+
+    f4_t acc[RT][NT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) acc[rt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    const h2_t m1056 = {(_Float16)-1056.0f, (_Float16)-1056.0f};
+
+    auto group = [&](const XRaw& r, int k, const WRaw& wc, const float (&dw)[RT][4]) {
+        h8_t Xh[2][NT], Xl[2][NT];
+        float ts[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            float f[16];
+#pragma unroll
+            for (int q = 0; q < 16; q++) f[q] = r.v[nt][q >> 2][q & 3];
+            float mx = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 16; q++) mx = fmaxf(mx, fabsf(f[q]));
+            // the largest of the token's 64 (lanes i, i + 16, i + 32, i + 48)
+            const uint32_t u = __float_as_uint(mx);
+            const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+            const uint32_t u2 = max(p[0], p[1]);   // (non-negative floats order as their bits)
+            const auto q2 = __builtin_amdgcn_permlane16_swap(u2, u2, false, false);
+            const int e = (int)(max(q2[0], q2[1]) >> 23);
+            const int fe = min(268 - e, 253);      // 2^(fe - 127) * mx in [2^14, 2^15)
+            const float sf = __uint_as_float((uint32_t)fe << 23);
+            ts[nt] = __uint_as_float((uint32_t)(254 - fe) << 23);
+#pragma unroll
+            for (int st = 0; st < 2; st++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float v = f[8 * st + j] * sf;
+                    const _Float16 hv = (_Float16)v;
+                    Xh[st][nt][j] = hv;
+                    Xl[st][nt][j] = (_Float16)(v - (float)hv);
+                }
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            const int sb = 2 * k + s;   // sub-block 8 h + 2 k + s
+            const _Float16 scf = (_Float16)(float)(int)(int8_t)byte_of(sb < 4 ? wc.sc[rt].x : wc.sc[rt].y, sb & 3);
+            const h2_t SC = {scf, scf};
+            f4_t S[NT];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                // codes of step 2 k + half: ql bytes 16 half + 8 (k & 1) + t, nibble
+                // k >> 1; qh bytes 8 half + t, bits 2 k .. 2 k + 1
+                const uint4 L = wc.ql[rt][half];
+                const uint32_t l0 = (k & 1) ? L.z : L.x, l1 = (k & 1) ? L.w : L.y;
+                const uint32_t h0 = half ? wc.qh[rt].z : wc.qh[rt].x, h1 = half ? wc.qh[rt].w : wc.qh[rt].y;
+                const uint32_t q0 = ((l0 >> (4 * (k >> 1))) & 0x0f0f0f0fu) | (((h0 >> (2 * k)) & 0x03030303u) << 4);
+                const uint32_t q1 = ((l1 >> (4 * (k >> 1))) & 0x0f0f0f0fu) | (((h1 >> (2 * k)) & 0x03030303u) << 4);
+                const h2_t v0 = bits_h2(__builtin_amdgcn_perm(kMagic, q0, kSelLo)) + m1056;
+                const h2_t v1 = bits_h2(__builtin_amdgcn_perm(kMagic, q0, kSelHi)) + m1056;
+                const h2_t v2 = bits_h2(__builtin_amdgcn_perm(kMagic, q1, kSelLo)) + m1056;
+                const h2_t v3 = bits_h2(__builtin_amdgcn_perm(kMagic, q1, kSelHi)) + m1056;
+                const h2_t w0 = v0 * SC, w1 = v1 * SC, w2 = v2 * SC, w3 = v3 * SC;
+                const h8_t Wa = __builtin_bit_cast(h8_t, make_uint4(h2_bits(w0), h2_bits(w1), h2_bits(w2), h2_bits(w3)));
+                const h8_t Wb = __builtin_bit_cast(
+                    h8_t, make_uint4(h2_bits(__builtin_elementwise_fma(v0, SC, -w0)), h2_bits(__builtin_elementwise_fma(v1, SC, -w1)),
+                                     h2_bits(__builtin_elementwise_fma(v2, SC, -w2)), h2_bits(__builtin_elementwise_fma(v3, SC, -w3))));
+                const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) S[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Wa, Xh[half][nt], half ? S[nt] : zero, 0, 0, 0);
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) S[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Wa, Xl[half][nt], S[nt], 0, 0, 0);
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) S[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Wb, Xh[half][nt], S[nt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    acc[rt][nt][v] = __builtin_fmaf(S[nt][v] * ts[nt], dw[rt][v], acc[rt][nt][v]);
+        }
+    };
+    XRaw x0, x1;
+    auto block = [&](int b, const WRaw& wc, WRaw& wn) {
+        const int bn = b + 4 < nb ? b + 4 : b;   // (the last block again at the end: no branch around the loads)
+        load_w(bn, wn);
+        float dw[RT][4];                         // d of rows 4 g + v
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            const float dl = hbits_to_f32(wc.dh[rt]);
+#pragma unroll
+            for (int v = 0; v < 4; v++) dw[rt][v] = __shfl(dl, 4 * g + v, 64);
+        }
+        load_x(b, 1, x1);
+        group(x0, 0, wc, dw);
+        load_x(b, 2, x0);
+        group(x1, 1, wc, dw);
+        load_x(b, 3, x1);
+        group(x0, 2, wc, dw);
+        load_x(bn, 0, x0);
+        group(x1, 3, wc, dw);
+    };
+    if (wave < nb) {
+        WRaw w0, w1;
+        load_w(wave, w0);
+        load_x(wave, 0, x0);
+        for (int b = wave; b < nb; b += 8) {
+            block(b, w0, w1);
+            if (b + 4 < nb) block(b + 4, w1, w0);
+        }
+    }
+    reduce_store<NT, RT>(acc, red, out, row0, tok0, d, m, vec, [&](int tok, int row) {
+        float sum = 0.0f;
+        for (int k = 0; k < n; k++)
+            sum = __builtin_fmaf(dequant_elem(w, 14, nblk, (size_t)row * nb + (k >> 8), k & 255), x[(size_t)tok * n + k], sum);
+        return sum;
+    });
+}
+
+// Tile shapes.  A tile's time does not depend on how many other workgroups
+// share the chip until a CU holds a second one, so a launch takes
+// ceil(workgroups / CUs) times the tile's own cost; the table's costs are the
+// times of one round in us (MI355X; bf16 over 2560 columns, where they follow
+// the bytes a tile loads, 2 NT + RT; Q6_K over 10240).  The cheapest shape is
+// taken; small batches get small tiles and so more workgroups.
+//   bf16 10752 x 2560, 512 tokens: 64 x 128 tiles 155 us, 64 x 64 198, 32 x 64
+//     223; 130 tokens 52 / 66 / 77; 37 tokens 52 / 32 / 41; 6 tokens 16 x 32
+//     17.6, 64 x 64 27.  fp32 matrix cores (64 x 32 tiles) before: 307, 106,
+//     55, 42.
+//   Q6_K 2560 x 10240, 512 tokens: 32 x 80 tiles 167 us, 16 x 16 498; 37
+//     tokens 16 x 32 38, 32 x 80 81; 6 tokens 16 x 16 23, 16 x 32 33.  fp32
+//     matrix cores before: 344, 94, 92.
+struct Tile {
+    int nt, rt, cost;
+    void (*launch)(const void* w, const float* x, float* o, int n, int d, int m);
+};
+
+template <int NT, int RT>
+void launch_bf16(const void* w, const float* x, float* o, int n, int d, int m) {
+    const int gx = (d + 16 * RT - 1) / (16 * RT), gy = (m + 16 * NT - 1) / (16 * NT);
+    hipLaunchKernelGGL((mm_batch_bf16_kernel<NT, RT>), dim3(gx * gy), dim3(256), 0, g4_stream(), (const uint16_t*)w, x, o, n,
+                       d, m, (int)(d % 4 == 0 && al16(o)));
+}
+template <int NT, int RT>
+void launch_q6(const void* w, const float* x, float* o, int n, int d, int m) {
+    const int gx = (d + 16 * RT - 1) / (16 * RT), gy = (m + 16 * NT - 1) / (16 * NT);
+    hipLaunchKernelGGL((mm_batch_q6_kernel<NT, RT>), dim3(gx * gy), dim3(256), 0, g4_stream(), (const uint8_t*)w, x, o, n, d,
+                       m, (int)(d % 4 == 0 && al16(o)));
+}
+
+const Tile kTilesBf16[] = {{1, 1, 3, launch_bf16<1, 1>},  {1, 2, 4, launch_bf16<1, 2>},  {2, 4, 8, launch_bf16<2, 4>},
+                           {4, 4, 12, launch_bf16<4, 4>}, {4, 6, 14, launch_bf16<4, 6>}, {4, 8, 16, launch_bf16<4, 8>}};
+const Tile kTilesQ6[] = {{1, 1, 25, launch_q6<1, 1>},
+                         {1, 2, 32, launch_q6<1, 2>},
+                         {2, 2, 52, launch_q6<2, 2>},
+                         {2, 4, 71, launch_q6<2, 4>},
+                         {2, 5, 81, launch_q6<2, 5>}};
+
+template <int N>
+const Tile& pick_tile(const Tile (&tiles)[N], int d, int m) {
+    const long long cus = g4_num_cus();
+    long long best = 0;
+    int at = -1;
+    for (int k = 0; k < N; k++) {
+        const Tile& t = tiles[k];
+        const long long wgs = (long long)((d + 16 * t.rt - 1) / (16 * t.rt)) * ((m + 16 * t.nt - 1) / (16 * t.nt));
+        const long long c = (wgs + cus - 1) / cus * t.cost;
+        if (at < 0 || c < best) best = c, at = k;
+    }
+    return tiles[at];
+}
+
+}  // namespace
+}  // namespace g4
+
+using namespace g4;
+
+extern "C" int g4_mm_batch_bf16_f32(float* o, const float* x, const void* w, int n, int d, int m) {
+    G4_CHECK_ARG(o && x && w, "g4_mm_batch_bf16_f32: null pointer");
+    G4_CHECK_ARG(n > 0 && n % 256 == 0 && d > 0 && m > 0 && (m + 31) / 32 <= 65535, "g4_mm_batch_bf16_f32: n=%d d=%d m=%d", n,
+                 d, m);
+    G4_CHECK_ARG(al16(x) && al16(w), "g4_mm_batch_bf16_f32: x and w must be 16-byte aligned");
+    // 64 rows x 32 tokens a workgroup (a sweep at the prompt's shape: 302 against 325 us at 64 x 16)
+    hipLaunchKernelGGL((mm_batch_f32_kernel<4, 2>), dim3((d + 63) / 64, (m + 31) / 32), dim3(256), 0, g4_stream(),
+                       (const uint16_t*)w, x, o, n, d, m);
+    return g4_check_launch("mm_batch_f32_kernel");
+}
+
+int g4_mm_batch_f32(float* o, const float* x, const void* w, int n, int d, int m, int type) {
+    const Tile& t = type == G4_BF16 ? pick_tile(kTilesBf16, d, m) : pick_tile(kTilesQ6, d, m);
+    t.launch(w, x, o, n, d, m);
+    return g4_check_launch(type == G4_BF16 ? "mm_batch_bf16_kernel" : "mm_batch_q6_kernel");
+}

@@ -1165,6 +1165,8 @@ static int mm_rows(g4e_model *m, float *o, const float *x, const Tensor *w, int 
         CK(g4_mm_batch_split(o, w->p, m->pf_xs, w->n, w->d, M, w->type));
         return 0;
     }
+    if (w->type == G4_BF16 && w->n % 256 == 0)
+        return g4_mm_batch_bf16_f32(o, x, w->p, w->n, w->d, M) ? lib_fail(G4_ERR_HIP, "g4_mm_batch_bf16_f32") : 0;
     return g4_mm_batch(o, x, w->p, w->n, w->d, M, w->type, m->pf_q8) ? lib_fail(G4_ERR_HIP, "g4_mm_batch") : 0;
 }
 

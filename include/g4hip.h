@@ -266,10 +266,14 @@ int g4_fold_gelu_mul_q8(const float *u, const void *q8, int n, const float *ple,
 /* m tokens through mm(o_t, x_t, w, n, d, type, q8, 0) (main.c:1669): Q4_K /
  * Q5_K quantize all rows into q8 (m * g4_q8K_row_stride(n) bytes) and take
  * g4_mm_batch_q8; Q6_K and BF16 with n a multiple of 256 and 16-byte aligned
- * x, w: one fp32 matrix-core GEMM on the fp32 activations (the reference's
- * dequantized fp32 weights, fp32 sums in another order; q8 unused);
+ * x, w: one matrix-core GEMM on the fp32 activations (split into 16-bit terms;
+ * the reference's dequantized weights, fp32 sums in another order; q8 unused);
  * otherwise the per-token GEMV m times. */
 int g4_mm_batch(float *o, const float *x, const void *w, int n, int d, int m, int type, void *q8);
+/* g4_mm_batch of a bf16 matrix (n a multiple of 256; x, w 16-byte aligned) with
+ * fp32 products and one fp32 sum per output in the order of K: the engine's
+ * prompt path (main.c:1529-1537 once per token), whose results keep their bits */
+int g4_mm_batch_bf16_f32(float *o, const float *x, const void *w, int n, int d, int m);
 /* Bytes of m split activation rows of n floats (n a multiple of 256): m * 4n
  * for the rows plus 4m for the per-row scale factors; 0 for bad sizes. */
 size_t g4_split_rows_bytes(int n, int m);

@@ -410,6 +410,88 @@ def test_mm_batch_f32_weights(lib, orc, qtype, n, d, m):
         assert (np.abs(got[t].astype(np.float64) - want) <= TOL * mag + 1e-30).all(), t
 
 
+@pytest.mark.parametrize("qtype", [14, 30])
+@pytest.mark.parametrize("n,d", [(256, 37), (768, 1000), (2560, 2560)])
+def test_mm_batch_f32_tiles(lib, qtype, n, d):
+    """Every tile shape of the Q6_K / bf16 GEMM on fp32 activations (batches of
+    1 to 600 tokens, rows that end inside a tile, an output that is only
+    4-byte aligned): a token's bits are the same in each, and within 1e-6 of
+    sum |w x| of the exact product (24-bit products and sums: 2^-22 an element
+    of the split, 2^-24 a sum, of which 1e-6 leaves a factor of three)."""
+    from g4 import DBuf, upload_quant
+    rng = np.random.default_rng(n + d + qtype)
+    raw = synth.rand_bf16(rng, d, n) if qtype == 30 else synth.rand_q6K(rng, d, n)
+    w = DBuf.from_array(lib, raw) if qtype == 30 else upload_quant(lib, raw, 14, n, d)
+    W = (raw.astype(np.uint32) << 16).view(np.float32) if qtype == 30 else kq.dequant_f64(raw.reshape(-1, 210), 14).astype(np.float32)
+    x = _acts(rng, 600, n)
+    x[7] *= np.float32(1e-30)
+    x[8] *= np.float32(1e30)
+    x[9, ::3] *= np.float32(1e6)
+    xd, out = DBuf.from_array(lib, x), DBuf(lib, 4 * (600 * d + 1))
+    W64, X64 = W.reshape(d, n).astype(np.float64), x.astype(np.float64)
+    want, mag = X64 @ W64.T, np.abs(X64) @ np.abs(W64).T
+    ref = None
+    for m in (600, 1, 5, 16, 17, 37, 64, 130, 257):
+        lib.g4_mm_batch(out.ptr + 4 * (m & 1), xd.ptr, w.ptr, n, d, m, qtype, None)
+        got = out.to_array(np.float32)[(m & 1):(m & 1) + m * d].reshape(m, d)
+        if ref is None:
+            ref = got.copy()
+        assert np.array_equal(got.view(np.uint32), ref[:m].view(np.uint32)), m
+    assert (np.abs(ref - want) <= 1e-6 * mag + 1e-37).all()
+
+
+@pytest.mark.parametrize("qtype", [14, 30])
+def test_mm_batch_f32_not_finite(lib, qtype):
+    """Infinities and NaN among the activations reach the outputs as in the
+    fp32 dot: an infinity where one meets a nonzero weight, NaN where it
+    meets a zero or an opposite infinity, nothing in the other tokens."""
+    from g4 import DBuf, upload_quant
+    rng = np.random.default_rng(5)
+    n, d, m = 512, 48, 21
+    raw = synth.rand_bf16(rng, d, n) if qtype == 30 else synth.rand_q6K(rng, d, n)
+    w = DBuf.from_array(lib, raw) if qtype == 30 else upload_quant(lib, raw, 14, n, d)
+    W = (raw.astype(np.uint32) << 16).view(np.float32) if qtype == 30 else kq.dequant_f64(raw.reshape(-1, 210), 14).astype(np.float32)
+    x = _acts(rng, m, n)
+    clean = DBuf.from_array(lib, x)
+    x[4, 300] = np.inf
+    x[6, 3] = -np.inf
+    x[8, [1, 400]] = np.inf, -np.inf
+    x[11, 511] = np.nan
+    x[13, 17] = 3.0e38
+    xd, out, out2 = DBuf.from_array(lib, x), DBuf(lib, 4 * m * d), DBuf(lib, 4 * m * d)
+    lib.g4_mm_batch(out.ptr, xd.ptr, w.ptr, n, d, m, qtype, None)
+    lib.g4_mm_batch(out2.ptr, clean.ptr, w.ptr, n, d, m, qtype, None)
+    got, base = out.to_array(np.float32).reshape(m, d), out2.to_array(np.float32).reshape(m, d)
+    with np.errstate(invalid="ignore"):
+        want = (x[:, None, :].astype(np.float64) * W.reshape(1, d, n)).sum(-1)
+    for t in range(m):
+        if t in (4, 6, 8, 11, 13):
+            assert np.array_equal(np.isnan(got[t]), np.isnan(want[t])), t
+            assert np.array_equal(np.sign(got[t][~np.isnan(got[t])]), np.sign(want[t][~np.isnan(want[t])])), t
+            assert np.array_equal(np.isinf(got[t]), np.abs(want[t]) > 3.4028235e38), t
+        else:
+            assert np.array_equal(got[t].view(np.uint32), base[t].view(np.uint32)), t
+
+
+def test_mm_batch_bf16_f32(lib, orc):
+    """The prompt path's bf16 GEMM: within 1e-5 of sum |w x| of mm_bf16
+    (main.c:1529-1537), each token's bits its own."""
+    from g4 import DBuf, G4Error
+    rng = np.random.default_rng(11)
+    n, d, m = 512, 1100, 45
+    raw, x = synth.rand_bf16(rng, d, n), _acts(rng, m, n)
+    w, xd, out = DBuf.from_array(lib, raw), DBuf.from_array(lib, x), DBuf(lib, 4 * m * d)
+    lib.g4_mm_batch_bf16_f32(out.ptr, xd.ptr, w.ptr, n, d, m)
+    got = out.to_array(np.float32).reshape(m, d).copy()
+    for t in (0, 1, 31, 32, m - 1):
+        want = orc.mm_bf16(x[t], raw, n, d)
+        assert (np.abs(got[t].astype(np.float64) - want) <= TOL * _mag_f32(raw, 30, n, d, x[t]) + 1e-30).all(), t
+    lib.g4_mm_batch_bf16_f32(out.ptr, xd.ptr + 4 * 9 * n, w.ptr, n, d, 7)
+    assert np.array_equal(out.to_array(np.float32)[:7 * d].view(np.uint32), got[9:16].reshape(-1).view(np.uint32))
+    with pytest.raises(G4Error):
+        lib.g4_mm_batch_bf16_f32(out.ptr, xd.ptr, w.ptr, 300, d, m)
+
+
 def test_mm_batch_wrapper(lib, orc):
     """g4_mm_batch for every type against the oracle per token: Q4_K / Q5_K
     through Q8_K rows (1e-5 of sum |terms| of the Q8_K dot), Q6_K and bf16
