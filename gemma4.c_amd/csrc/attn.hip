@@ -1575,6 +1575,333 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
     }
 }
 
+// ---- query rows at head_dim 512 on split fp16 products -----------------------
+// attn_rows_mfma_kernel<512>'s partials on split fp16 products (as in
+// attn_rows_h16_kernel, whose registers do not suffice at 512): eight waves a
+// workgroup, wave (h, half) takes q head 4 kvh + h and dims 256 half .. + 255,
+// for the scores (the two halves' sums meet in LDS) and for the output, so a
+// wave holds 64 registers of q and 64 of o.  32 keys a tile: both products use
+// v_mfma_f32_16x16x32_f16.
+// Range: the four K rows that a wave stages, its four V rows and every half q
+// row are scaled by the power of two that brings their largest element into
+// [2^14, 2^15) before the split (an element is then within 2^-22 of its value or
+// 2^-39 of that largest), so any finite fp32 input keeps its range.  The K
+// factor multiplies the scores; the V factor goes into its keys' weights, which
+// are kept relative to the largest factor met so far (o is scaled down when a
+// larger one comes).
+// LDS: K as rows of 512 hi, 512 lo (2080 bytes a row: conflict-free 16-byte
+// reads); V transposed, a 128-byte row per dim of eight 16-byte slots, slot (hl,
+// g) at (g + 4 hl) ^ (dim / 2 & 7): the keys 4g .. 4g + 3 of both 16-key halves,
+// the order in which a lane holds its weights.  Wave w stages keys 4w .. 4w + 3
+// whole, so their largest element is a reduction within the wave.
+// Two barriers a tile: V is split and staged between the score products, the
+// next tile's K between the output products, and each row's loads take the
+// registers of a row just staged (all 64 at once spilled: 470 us at the size
+// below).  512 rows at positions 7680 .. 8191, 16 chunks: 872 us on the fp32
+// matrix cores; here 545 with the addresses behind branches (each load waited
+// for all before it), 465 without, 419 with operands read ahead of their
+// products, 360 with the splits between the products.  What is left is VALU
+// issue (half of the time) and the matrix cores (a quarter), which a wave
+// overlaps only in part.
+constexpr int kR5Keys = 32, kR5KRow = 2080;
+typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) const f2_t g4_gf2_t;
+typedef _Float16 ah2_t __attribute__((ext_vector_type(2)));
+
+// x sf and y sf as fp16 hi + lo (round to nearest; x sf - hi is exact)
+__device__ __forceinline__ void split2(float x, float y, float sf, ah2_t& hi, ah2_t& lo) {
+    hi = __builtin_convertvector((f2_t{x * sf, y * sf}), ah2_t);
+    lo = __builtin_convertvector((f2_t{__builtin_fmaf(x, sf, -(float)hi[0]), __builtin_fmaf(y, sf, -(float)hi[1])}), ah2_t);
+}
+// max(|x|, |y|, m) in one instruction (fmaxf on loaded values is three)
+__device__ __forceinline__ float max3_abs(float x, float y, float m) {
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(x), "v"(y), "v"(m));
+    return r;
+}
+// e^x for x <= kRowsLazy, 0 below the smallest normal number: 2^(x log2 e) with
+// the product's rounding error put back to first order (within 2 ulp)
+__device__ __forceinline__ float exp_le(float x) {
+    const float t = x * 1.44269504f;
+    const float r = __builtin_fmaf(x, 1.92596303e-8f, __builtin_fmaf(x, 1.44269504f, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(e, r * 0.693147181f, e);
+}
+__device__ __forceinline__ ah4_t join4(ah2_t a, ah2_t b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3); }
+
+// exponent field f of the scale 2^(f - 127) that brings mx into [2^14, 2^15)
+// (clamped so that 16 times its inverse 2^(127 - f) inverts again)
+__device__ __forceinline__ int scale_field(float mx) { return max(1, min(268 - (int)(__float_as_uint(mx) >> 23), 248)); }
+__device__ __forceinline__ float field_to_scale(int f) { return __uint_as_float((uint32_t)f << 23); }
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void attn_rows512_kernel(AttnArgs a) {
+    constexpr int HD = 512;
+    __shared__ __align__(16) uint8_t ks[kR5Keys * kR5KRow];
+    __shared__ __align__(16) uint8_t vs[HD * 128];
+    __shared__ __align__(16) float tsk[8], tsv[8];
+    __shared__ __align__(16) f4_t ex[8][2][64];
+    const int c = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, j = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave & 1;
+    const int head = kvh * kRowsKVM + (wave >> 1);
+    const int M = a.qrows;
+    const int z0 = 16 * rb, z1 = min(z0 + 16, M) - 1;
+    const int lo = a.window > 0 ? max(0, a.p0 + z0 + 1 - a.window) : 0;
+    const int hi = a.p0 + z1;
+    const int cs = ((hi - lo + a.G) / a.G + kR5Keys - 1) / kR5Keys * kR5Keys;   // whole tiles
+    const int cb = lo + c * cs, ce = min(cb + cs, hi + 1);
+    const int z = z0 + j;
+    const int qp = a.p0 + z;
+    const int qlo = a.window > 0 ? max(0, qp + 1 - a.window) : 0;
+    const int qend = min(qp, ce - 1);
+
+    // this wave's rows of a tile: keys 4 wave + r, K as float4 (dims 4 lane, 256 +
+    // 4 lane), V as float2 (dims 128 k + 2 lane); past the chunk the last
+    // position again (its weight is 0)
+    f4_t kr[4][2];
+    f2_t vr[4][4];
+    const int tl = ce - 1;
+    const unsigned ring = a.ring > 0 ? (unsigned)a.ring : 0x7fffffffu;
+    // byte address of row r (selects, no branch: a load behind one would wait
+    // for every load before it)
+    auto row_of = [&](int t0, int r, const float* cache, const float* own) {
+        const int tf = min(t0 + 4 * wave, tl), t = min(t0 + 4 * wave + r, tl);
+        unsigned slot = (unsigned)tf % ring + (unsigned)(t - tf);
+        slot = slot >= ring ? slot - ring : slot;
+        const bool mine = t >= a.p0;
+        const size_t off = (size_t)(mine ? (unsigned)(t - a.p0) : slot) * a.kv_stride + (size_t)kvh * HD;
+        return (mine ? (uintptr_t)own : (uintptr_t)cache) + 4 * off;
+    };
+    auto load_k = [&](int t0, int r) {
+        const uintptr_t p = row_of(t0, r, a.kc, a.kchunk);
+#pragma unroll
+        for (int k = 0; k < 2; k++) kr[r][k] = reinterpret_cast<const g4_gf4_t*>(p)[lane + 64 * k];
+    };
+    auto load_v = [&](int t0, int r) {
+        const uintptr_t p = row_of(t0, r, a.vc, a.vchunk);
+#pragma unroll
+        for (int k = 0; k < 4; k++) vr[r][k] = reinterpret_cast<const g4_gf2_t*>(p)[lane + 64 * k];
+    };
+    // staging, in parts that the products below are interleaved with
+    float ksf, vsf;
+    auto scale_k = [&]() {
+        float mx = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) mx = max3_abs(kr[r][k][2], kr[r][k][3], max3_abs(kr[r][k][0], kr[r][k][1], mx));
+        const int f = scale_field(wave_max(mx));
+        ksf = field_to_scale(f);
+        if (lane == 0) tsk[wave] = field_to_scale(254 - f);
+    };
+    auto stage_k = [&](int r, int k) {
+        uint8_t* row = ks + (4 * wave + r) * kR5KRow + 8 * lane;
+        ah2_t h0, l0, h1, l1;
+        split2(kr[r][k][0], kr[r][k][1], ksf, h0, l0);
+        split2(kr[r][k][2], kr[r][k][3], ksf, h1, l1);
+        *reinterpret_cast<ah4_t*>(row + 512 * k) = join4(h0, h1);
+        *reinterpret_cast<ah4_t*>(row + 512 * k + 1024) = join4(l0, l1);
+    };
+    auto scale_v = [&]() {
+        float mx = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) mx = max3_abs(vr[r][k][0], vr[r][k][1], mx);
+        const int f = scale_field(wave_max(mx));
+        vsf = field_to_scale(f);
+        if (lane == 0) tsv[wave] = field_to_scale(254 - f);
+    };
+    const int kt4 = wave >> 2, kg4 = wave & 3;   // keys 16 kt4 + 4 kg4 + r
+    auto stage_v = [&](int k, int x) {
+        const int dim = 128 * k + 2 * lane + x, sw = lane & 7;   // sw = dim / 2 & 7
+        ah2_t h0, l0, h1, l1;
+        split2(vr[0][k][x], vr[1][k][x], vsf, h0, l0);
+        split2(vr[2][k][x], vr[3][k][x], vsf, h1, l1);
+        *reinterpret_cast<ah4_t*>(vs + dim * 128 + 16 * (kg4 ^ sw) + 8 * kt4) = join4(h0, h1);
+        *reinterpret_cast<ah4_t*>(vs + dim * 128 + 16 * ((kg4 + 4) ^ sw) + 8 * kt4) = join4(l0, l1);
+    };
+
+    // q of row j, dims 256 half + 32 s + 8 g .. + 7
+    ah8_t qh[8], ql[8];
+    float tsq;
+    {
+        const float* qrow = a.q + (size_t)min(z, M - 1) * a.n_heads * HD + (size_t)head * HD + 256 * half + 8 * g;
+        float mx = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+#pragma unroll
+            for (int t = 0; t < 8; t++) mx = fmaxf(mx, fabsf(qrow[32 * s + t]));
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const int f = scale_field(mx);
+        const float sf = field_to_scale(f);
+        tsq = field_to_scale(254 - f);
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                const float v = qrow[32 * s + t] * sf;
+                const _Float16 h = split_hi(v);
+                qh[s][t] = h;
+                ql[s][t] = split_lo(v, h);
+            }
+    }
+
+    float m = -INFINITY, lsum = 0.0f;   // lsum: this lane's keys only (summed over the groups at the end)
+    float E = field_to_scale(6);        // the largest V factor met
+    f4_t o[16];
+#pragma unroll
+    for (int b = 0; b < 16; b++) o[b] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if (cb < ce) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) load_k(cb, r);
+        scale_k();
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            stage_k(r, 0);
+            stage_k(r, 1);
+            load_v(cb, r);
+        }
+    }
+    for (int t0 = cb; t0 < ce; t0 += kR5Keys) {
+        lds_sync();   // K is staged, V is free
+        // this half's scores of keys 16 t + 4 g + r and row j (a step's operands
+        // are read before the products of the step before)
+        f4_t sh[2], sx[2];
+        ah8_t Ah[2][2], Al[2][2];
+        const uint8_t* kp = ks + j * kR5KRow + 512 * half + 16 * g;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            sh[t] = sx[t] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            Ah[0][t] = *reinterpret_cast<const ah8_t*>(kp + 16 * t * kR5KRow);
+            Al[0][t] = *reinterpret_cast<const ah8_t*>(kp + 16 * t * kR5KRow + 1024);
+        }
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int cu = s & 1;
+            if (s < 7) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    Ah[cu ^ 1][t] = *reinterpret_cast<const ah8_t*>(kp + 16 * t * kR5KRow + 64 * (s + 1));
+                    Al[cu ^ 1][t] = *reinterpret_cast<const ah8_t*>(kp + 16 * t * kR5KRow + 64 * (s + 1) + 1024);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                sh[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[cu][t], qh[s], sh[t], 0, 0, 0);
+                sx[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[cu][t], ql[s], sx[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++) sx[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[cu][t], qh[s], sx[t], 0, 0, 0);
+            if (s == 3) scale_v();
+            if (s >= 4) {   // this tile's V rows; the next tile's K loads take their registers
+                stage_v(s - 4, 0);
+                stage_v(s - 4, 1);
+                load_k(t0 + kR5Keys, s - 4);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const float k4[2] = {tsk[g], tsk[4 + g]};   // of keys 16 t + 4 g + r
+#pragma unroll
+        for (int t = 0; t < 2; t++) ex[wave][t][lane] = (sh[t] + sx[t]) * tsq;
+        lds_sync();   // both halves' sums, V is staged, K is free
+        const float v4[2] = {tsv[g], tsv[4 + g]};
+        float sv[8], mt = -INFINITY, et = fmaxf(v4[0], v4[1]);
+        bool val[8];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const f4_t sc = (ex[wave & ~1][t][lane] + ex[wave | 1][t][lane]) * k4[t];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int kt = t0 + 16 * t + 4 * g + r, e = 4 * t + r;
+                val[e] = (kt >= qlo) & (kt <= qend);
+                sv[e] = val[e] ? a.scale * sc[r] : -INFINITY;
+                mt = fmaxf(mt, sv[e]);
+            }
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        et = fmaxf(et, __shfl_xor(et, 16, 64));
+        et = fmaxf(et, __shfl_xor(et, 32, 64));   // the tile's largest factor, the same in every lane
+        const bool up = mt > m + kRowsLazy;   // as in attn_rows_mfma_kernel
+        const float mn = up ? mt : m;
+        const float En = fmaxf(E, et);
+        if (__ballot(up || En != E)) {
+            const float alpha = !up ? 1.0f : m == -INFINITY ? 0.0f : expf(m - mn);
+            lsum *= alpha;
+            const float beta = alpha * (E / En);   // (E / En: powers of two)
+#pragma unroll
+            for (int b = 0; b < 16; b++) o[b] *= beta;
+        }
+        float p[8], ps = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            p[e] = exp_le(val[e] ? sv[e] - mn : -200.0f);   // (e^-200 is 0)
+            ps += p[e];
+        }
+        lsum += ps;
+        m = mn;
+        E = En;
+        ah8_t Ph, Pl;
+        const float u16 = field_to_scale(258 - (int)(__float_as_uint(E) >> 23));   // 16 / E
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {   // <= 16 e^kRowsLazy
+            ah2_t h, l;
+            split2(p[e], p[e + 1], v4[e >> 2] * u16, h, l);
+            Ph[e] = h[0];
+            Ph[e + 1] = h[1];
+            Pl[e] = l[0];
+            Pl[e + 1] = l[1];
+        }
+        // O^T += V^T . P^T over the 32 keys, operands read two blocks ahead
+        const int sw = (j >> 1) & 7;
+        const uint8_t* vph = vs + (256 * half + j) * 128 + 16 * (g ^ sw);
+        const uint8_t* vpl = vs + (256 * half + j) * 128 + 16 * ((g + 4) ^ sw);
+        ah8_t Vh[3], Vl[3];
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            Vh[b] = *reinterpret_cast<const ah8_t*>(vph + 2048 * b);
+            Vl[b] = *reinterpret_cast<const ah8_t*>(vpl + 2048 * b);
+        }
+#pragma unroll
+        for (int b = 0; b < 16; b++) {
+            if (b < 14) {
+                Vh[(b + 2) % 3] = *reinterpret_cast<const ah8_t*>(vph + 2048 * (b + 2));
+                Vl[(b + 2) % 3] = *reinterpret_cast<const ah8_t*>(vpl + 2048 * (b + 2));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Vh[b % 3], Pl, o[b], 0, 0, 0);
+            o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Vl[b % 3], Ph, o[b], 0, 0, 0);
+            o[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Vh[b % 3], Ph, o[b], 0, 0, 0);
+            // the next tile's K rows; its V loads take their registers
+            if (b == 0) scale_k();
+            if (b >= 1 && b <= 8) stage_k((b - 1) >> 1, (b - 1) & 1);
+            if (b >= 2 && b <= 8 && !(b & 1)) load_v(t0 + kR5Keys, (b >> 1) - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    lsum += __shfl_xor(lsum, 16, 64);
+    lsum += __shfl_xor(lsum, 32, 64);
+    if (z < M) {
+        // o[b][r] is dim 256 half + 16 b + 4 g + r of row z
+        float* pp = a.part + (size_t)z * a.part_z + ((size_t)head * a.G + c) * (HD + 2);
+        const float un = E * (1.0f / 16.0f);
+#pragma unroll
+        for (int b = 0; b < 16; b++) {
+            float* q = pp + 256 * half + 16 * b + 4 * g;
+            *reinterpret_cast<float2*>(q) = make_float2(o[b][0] * un, o[b][1] * un);
+            *reinterpret_cast<float2*>(q + 2) = make_float2(o[b][2] * un, o[b][3] * un);
+        }
+        if (g == 0 && half == 0) {
+            pp[HD] = m;
+            pp[HD + 1] = lsum;
+        }
+    }
+}
+
 // partial kernel LDS: work region + (max, sum) pairs [+ this position's K, V]
 size_t attn_lds(int hd, int kvm, bool fused) {
     return 4 * (fused ? (size_t)attn_new_kv_off(hd, kvm) + 2 * (size_t)hd
@@ -1622,6 +1949,16 @@ void launch_merge(const AttnArgs& a, const dim3& grid) {
     else hipLaunchKernelGGL((attn_merge_kernel<HD, 128>), grid, dim3(256), 0, g4_stream(), a);
 }
 
+// head_dim 512 over query rows: attn_rows512_kernel (us, launch and merge,
+// against attn_rows_mfma_kernel<512>: 37 rows at position 0 21.7 / 26.6, 511 rows
+// 48.5 / 77, 512 rows at 1536 165 / 329, at 7680 360 / 872, 4 rows at 7000 63 /
+// 172; error against 64 bits 1.4e-7 .. 3.5e-7 / 1.7e-7 .. 5.0e-7).  The fp32 kernel
+// keeps the rows that are quantized on the spot (q8) within the first 1024
+// positions: an engine's prompt of that length goes through 8-bit codes in every
+// layer, where another order of sums moves some code by one and the model carries
+// it on, so it keeps the bits, and the tokens, it had.
+constexpr int kRowsQ8Keys = 1024;
+
 int launch_attn(const AttnArgs& a) {
     const int kvm = a.n_heads / a.n_kv;
     const int zq = a.qrows > 0 ? a.qrows : 1;
@@ -1635,11 +1972,11 @@ int launch_attn(const AttnArgs& a) {
             hipLaunchKernelGGL(attn_rows_h16_kernel<256>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
             launch_merge<256>(a, dim3(a.n_heads, 1, zq));
         } else {
-            // (the split form needs 35 VGPRs more than a wave has at hd 512)
-            hipLaunchKernelGGL(attn_rows_mfma_kernel<512>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
+            if (!a.q8 || a.p0 + a.qrows > kRowsQ8Keys) hipLaunchKernelGGL(attn_rows512_kernel, rgrid, dim3(512), 0, g4_stream(), a);
+            else hipLaunchKernelGGL(attn_rows_mfma_kernel<512>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
             launch_merge<512>(a, dim3(a.n_heads, 2, zq));
         }
-        return g4_check_launch("attn_rows_h16_kernel/attn_rows_mfma_kernel/attn_merge_kernel");
+        return g4_check_launch("attn_rows kernel/attn_merge_kernel");
     }
     if (attn_chunk_lds(a.hd, kp) <= 65536) {
         // no out: the partials only, merged by the caller (g4_mm_attn_merge)

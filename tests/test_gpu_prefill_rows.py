@@ -348,3 +348,50 @@ def test_attn_decode_rows_peaked_small(lib, orc, hd):
         p = np.exp(s - s.max())
         frac.append(np.mean((p > 1e-3) & (p < 1e-1)))
     assert np.mean(frac) > 0.2, np.mean(frac)
+
+
+ROWS512_CASES = [
+    # p0, m, G, window, ring, scale of K, scale of V
+    (0, 1, 1, 0, 0, 1.0, 1.0),             # a single row and key
+    (0, 37, 3, 0, 0, 1.0, 1.0),            # rows that end inside a 16-row block, chunks inside a tile
+    (995, 61, 16, 0, 0, 1.0, 1.0),         # cache and chunk rows in one tile, chunks of whole tiles
+    (700, 50, 4, 300, 300, 1.0, 1.0),      # a wrapped ring, windows that start inside a tile
+    (100, 33, 16, 0, 0, 1e-5, 1e-5),       # K and V far below fp16's range unless scaled
+    (64, 40, 2, 0, 0, 1e5, 1e6),           # ... and above it
+]
+
+
+@pytest.mark.parametrize("p0,m,G,window,ring,ks,vs", ROWS512_CASES)
+def test_attn_decode_rows_512(lib, p0, m, G, window, ring, ks, vs):
+    """head_dim 512 on split fp16 products against the attention in 64 bits:
+    every element is held to 2^-22, so a score of |s| <= 6 is off by less than
+    2^-20 and the output by less than 1e-5 of max|o|.  Key rows differ in size by
+    factors up to 2^8, so that the per-row-group scales change between tiles;
+    rows no query may read hold NaN."""
+    hd, n_heads, n_kv = 512, 8, 2
+    rng = np.random.default_rng(p0 + m + G)
+    kvd, T = n_kv * hd, p0 + m
+    V = rng.standard_normal((T, kvd)) * vs * 2.0 ** rng.integers(0, 8, (T, 1))
+    K = (rng.standard_normal((T, kvd)) * ks).astype(np.float32)
+    V, q = V.astype(np.float32), (rng.standard_normal((m, n_heads * hd)) * hd ** -0.5 / ks).astype(np.float32)
+    slots = ring if ring else T
+    kc, vc = np.full((slots, kvd), np.nan, np.float32), np.full((slots, kvd), np.nan, np.float32)
+    for t in range(max(0, p0 - ring) if ring else 0, p0):
+        kc[t % slots], vc[t % slots] = K[t], V[t]
+    pad = np.full((2, kvd), np.nan, np.float32)
+    kch, vch = np.concatenate([K[p0:], pad]), np.concatenate([V[p0:], pad])
+    part = empty(lib, m * lib.L.g4_attn_part_bytes(n_heads, hd, G))
+    out = empty(lib, 4 * m * n_heads * hd)
+    qd, kcd, vcd, kchd, vchd = dbuf(lib, q), dbuf(lib, kc), dbuf(lib, vc), dbuf(lib, kch), dbuf(lib, vch)
+    lib.g4_attn_decode_rows(qd.ptr, kcd.ptr, vcd.ptr, kchd.ptr, vchd.ptr, kvd, ring, p0, m, window, n_heads, n_kv, hd,
+                            F(1.0), G, part.ptr, out.ptr, None)
+    got = out.to_array(np.float32).reshape(m, n_heads, hd)
+    K64, V64, q64 = (a.astype(np.float64).reshape(-1, h, hd) for a, h in ((K, n_kv), (V, n_kv), (q, n_heads)))
+    for z in range(m):
+        pos = p0 + z
+        t0 = max(0, pos + 1 - window) if window else 0
+        for h in range(n_heads):
+            s = K64[t0:pos + 1, h // 4] @ q64[z, h]
+            w = np.exp(s - s.max())
+            want = (w / w.sum()) @ V64[t0:pos + 1, h // 4]
+            assert np.abs(got[z, h] - want).max() <= 1e-5 * np.abs(want).max(), (z, h)
