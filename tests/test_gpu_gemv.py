@@ -318,6 +318,33 @@ def test_mm_single_block_quantizes_inside(lib, orc, qtype):
     assert download_q8(lib, q8, n).tobytes() == q8h.tobytes()
 
 
+@pytest.mark.parametrize("qtype", [12, 13])
+@pytest.mark.parametrize("n", [2048, 2560, 4096])
+@pytest.mark.parametrize("d", [1, 37, 2560, 2561])
+def test_mm_quantizes_inside(lib, orc, qtype, n, d):
+    """g4_mm that quantizes x in its own launch (up to 2560 rows), and in a
+    launch before: the output and the stored Q8_K of quantize_row_q8_K +
+    mm_quant_dot_rows, bit for bit, also where o lies on x."""
+    from g4 import DBuf, upload_quant
+    rng = np.random.default_rng(n + d + qtype)
+    x = rng.standard_normal(n).astype(np.float32)
+    x[256:512] = 0.0
+    w = upload_quant(lib, synth.rand_kquant(rng, qtype, d, n), qtype, n, d)
+    xd, want = dbuf(lib, x), DBuf(lib, 4 * d)
+    q8, q8b = DBuf(lib, lib.L.g4_q8K_bytes(n)), DBuf(lib, lib.L.g4_q8K_bytes(n))
+    lib.g4_quantize_row_q8_K(xd.ptr, q8.ptr, n)
+    lib.g4_mm_quant_dot_rows(want.ptr, w.ptr, n, d, qtype, q8.ptr)
+    want = want.to_array(np.uint32)
+    out = DBuf(lib, 4 * d)
+    lib.g4_mm(out.ptr, xd.ptr, w.ptr, n, d, qtype, q8b.ptr, 0)
+    assert np.array_equal(out.to_array(np.uint32), want)
+    assert np.array_equal(xd.to_array(np.float32), x)
+    assert download_q8(lib, q8b, n).tobytes() == download_q8(lib, q8, n).tobytes()
+    if d <= n:
+        lib.g4_mm(xd.ptr, xd.ptr, w.ptr, n, d, qtype, q8b.ptr, 0)
+        assert np.array_equal(xd.to_array(np.uint32)[:d], want)
+
+
 def rel_err(got, want):
     want = np.asarray(want, np.float64)
     return float(np.max(np.abs(np.asarray(got, np.float64) - want)) / max(np.max(np.abs(want)), 1e-30))
