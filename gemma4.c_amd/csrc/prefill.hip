@@ -360,6 +360,185 @@ void launch_mm_batch8(const KqSegs& sg, const uint8_t* q8, int nb, int m) {
                        sg, q8, nb, m);
 }
 
+// ---- Q4_K / Q5_K with the waves over K (mm_batch_kq8w_kernel) ----------------
+// mm_batch_kq8_kernel runs a tile's blocks one after the other with one block
+// of loads in flight: about 2 us a block whatever the work, which is the whole
+// time when the tiles do not fill the chip.  Here the NWV waves of a workgroup
+// take one block each of the same 32 rows x 32 tokens, everything in flight at
+// once; each stages its block's codes for itself (no barrier), forms the same
+// per-block term u = fma(d, S_b, -(dmin M_b)) as MODE 1 above and leaves it in
+// LDS, and after one barrier the terms of the round's blocks are folded in block
+// order, out = fma(d_t, u_b, out): mm_batch_kq8_kernel's bits.  More blocks than
+// waves take several rounds.
+// A load instruction costs the L1 four cycles for every 128-byte line that it
+// touches (measured: 16 rows x 64 bytes 38 bytes/ns a CU, whole lines 74), so
+// codes of weights and activations are read as whole lines, eight lanes a line,
+// and brought into operand order through LDS.
+// LDS of a wave: the weight codes until it has read them, then the activation
+// codes, then the terms.
+constexpr int kKqwTermRow = 33;                 // floats of a token's row of terms
+constexpr int kKqwWave = 32 * kKq8Tok;
+static_assert(kKqwWave >= 4 * 32 * kKqwTermRow && kKqwWave >= 32 * 128, "terms and weight codes fit");
+
+template <bool Q5, int NWV>
+__global__ __launch_bounds__(64 * NWV) void mm_batch_kq8w_kernel(const KqSegs sg, const uint8_t* __restrict__ q8, int nb,
+                                                                 int m) {
+    typedef int i4v_t __attribute__((ext_vector_type(4)));
+    typedef int i16v_t __attribute__((ext_vector_type(16)));
+    constexpr int NTH = 64 * NWV, EPT = (1024 + NTH - 1) / NTH;   // outputs a thread folds
+    __shared__ __align__(16) uint8_t sX[NWV][kKqwWave];
+    __shared__ float sD[NWV][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 31, kg = lane >> 5;
+    int bx, by;
+    xcd_tile((m + 31) / 32, bx, by);
+    int seg = 0;
+#pragma unroll
+    for (int k = 1; k < kMaxSegs; k++)
+        if (k < sg.n && bx >= sg.g0[k]) seg = k;
+    const uint8_t* __restrict__ w = sg.w[seg];
+    const int d = sg.d[seg];
+    float* __restrict__ out = sg.o[seg];
+    const int row0 = (bx - sg.g0[seg]) * 32, tok0 = by * 32;
+    const size_t nblk = (size_t)d * nb;
+    const int hdr_off = (int)((Q5 ? 160 : 128) * nblk), qh_off = (int)(128 * nblk);
+    const int q8row = (int)(((size_t)nb * 292 + 63) & ~(size_t)63);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, (int)(hdr_off + 16 * nblk), kBufWord3);
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void*)q8, (short)0, (int)((size_t)m * q8row), kBufWord3);
+    const int rB = min(row0 + i, d - 1) * nb;              // this lane's weight row and token
+    const int tB = min(tok0 + i, m - 1) * q8row;
+    const int vhdr = hdr_off + rB * 16, vqh = qh_off + rB * 32 + 16 * kg;
+    const int vbs = tB + (int)q8k_bsums_off(nb) + 8 * kg, vd = tB + (int)q8k_d_off(nb);
+    int vw[4], vx[8];                                      // whole lines: weights 8 rows, activations 4 tokens
+#pragma unroll
+    for (int q = 0; q < 4; q++) vw[q] = min(row0 + 8 * q + (lane >> 3), d - 1) * nb * 128 + 16 * (lane & 7);
+#pragma unroll
+    for (int q = 0; q < 8; q++) vx[q] = min(tok0 + 4 * q + (lane >> 4), m - 1) * q8row + 16 * (lane & 15);
+
+    float acc[EPT];
+#pragma unroll
+    for (int e = 0; e < EPT; e++) acc[e] = 0.0f;
+    for (int b0 = 0; b0 < nb; b0 += NWV) {
+        const int b = min(b0 + wave, nb - 1);              // (a wave past the end repeats the last block, unused)
+        uint4 wq[4], xq[8], qhv = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; q++) wq[q] = buf_load16(rw, vw[q], b * 128);
+        const uint4 hdr = buf_load16(rw, vhdr, b * 16);
+        if (Q5) qhv = buf_load16(rw, vqh, b * 32);
+#pragma unroll
+        for (int q = 0; q < 8; q++) xq[q] = buf_load16(rq, vx[q], b * 256);
+        const uint2 c1 = buf_load8(rq, vbs, b * 32), c2 = buf_load8(rq, vbs + 16, b * 32);   // bsums 4 kg .., 8 + 4 kg ..
+        const float yd = __uint_as_float(buf_load4(rq, vd, b * 4));
+        if (b0) lds_barrier();                             // the last round's terms have been read
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int rr = 8 * q + (lane >> 3);
+            *reinterpret_cast<uint4*>(sX[wave] + rr * 128 + 16 * ((lane & 7) ^ ((rr >> 1) & 7))) = wq[q];
+        }
+        uint4 W[4];                                        // this lane's 64 code bytes: words 16 kg .. 16 kg + 15
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            W[q] = *reinterpret_cast<const uint4*>(sX[wave] + i * 128 + 16 * ((4 * kg + q) ^ ((i >> 1) & 7)));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        // device words 4u .. 4u + 3 (u = lane & 15): l' = u / 2, h = u & 1, jj = 0 .. 3
+        // -> sub-block 2 jj + h, positions 4 l' .. 4 l' + 3
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            uint8_t* dst = sX[wave] + (4 * q + (lane >> 4)) * kKq8Tok + 32 * (lane & 1) + 4 * ((lane & 15) >> 1);
+            *reinterpret_cast<uint32_t*>(dst) = xq[q].x;
+            *reinterpret_cast<uint32_t*>(dst + 64) = xq[q].y;
+            *reinterpret_cast<uint32_t*>(dst + 128) = xq[q].z;
+            *reinterpret_cast<uint32_t*>(dst + 192) = xq[q].w;
+        }
+        if (!kg) sD[wave][i] = yd;
+        uint32_t sc_lo, sc_hi, mn_lo, mn_hi;
+        unpack_scales(hdr.y, hdr.z, hdr.w, sc_lo, sc_hi, mn_lo, mn_hi);
+        i16v_t izero;
+        f16v_t zero;
+#pragma unroll
+        for (int v = 0; v < 16; v++) izero[v] = 0, zero[v] = 0.0f;
+        int SI[16];
+        const uint8_t* at0 = sX[wave] + i * kKq8Tok + 16 * kg;
+#pragma unroll
+        for (int sb = 0; sb < 8; sb++) {
+            const int c = sb >> 1, h = sb & 1;
+            uint32_t cw[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t word = c == 0 ? W[q].x : c == 1 ? W[q].y : c == 2 ? W[q].z : W[q].w;
+                uint32_t v = h ? (word >> 4) & 0x0f0f0f0fu : word & 0x0f0f0f0fu;
+                if (Q5) {
+                    const uint32_t hw = q == 0 ? qhv.x : q == 1 ? qhv.y : q == 2 ? qhv.z : qhv.w;
+                    v |= ((hw >> sb) & 0x01010101u) << 4;
+                }
+                cw[q] = v;
+            }
+            const i4v_t B = {(int)cw[0], (int)cw[1], (int)cw[2], (int)cw[3]};
+            const int scv = byte_of(sb < 4 ? sc_lo : sc_hi, sb & 3);
+            const i4v_t A = *reinterpret_cast<const i4v_t*>(at0 + 32 * sb);
+            const i16v_t Z = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, izero, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 16; v++) SI[v] = (sb == 0 ? 0 : SI[v]) + __mul24(scv, Z[v]);
+        }
+        const h4_t A1 = {(_Float16)(int16_t)(c1.x & 0xffffu), (_Float16)(int16_t)(c1.x >> 16),
+                         (_Float16)(int16_t)(c1.y & 0xffffu), (_Float16)(int16_t)(c1.y >> 16)};
+        const h4_t A2 = {(_Float16)(int16_t)(c2.x & 0xffffu), (_Float16)(int16_t)(c2.x >> 16),
+                         (_Float16)(int16_t)(c2.y & 0xffffu), (_Float16)(int16_t)(c2.y >> 16)};
+        const int msh = 16 * kg;
+        const _Float16 m0 = (_Float16)(float)((mn_lo >> msh) & 0xffu), m1 = (_Float16)(float)((mn_lo >> (msh + 8)) & 0xffu);
+        const _Float16 m4 = (_Float16)(float)((mn_hi >> msh) & 0xffu), m5 = (_Float16)(float)((mn_hi >> (msh + 8)) & 0xffu);
+        const h4_t Bm1 = {m0, m0, m1, m1}, Bm2 = {m4, m4, m5, m5};
+        f16v_t M = __builtin_amdgcn_mfma_f32_32x32x8f16(A1, Bm1, zero, 0, 0, 0);
+        M = __builtin_amdgcn_mfma_f32_32x32x8f16(A2, Bm2, M, 0, 0, 0);
+        const float dx = hbits_to_f32(hdr.x & 0xffffu), dmx = hbits_to_f32(hdr.x >> 16);
+        // (the wave's reads of its codes are done: the terms take their place)
+        float* term = reinterpret_cast<float*>(sX[wave]);
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            term[(8 * (v >> 2) + 4 * kg + (v & 3)) * kKqwTermRow + i] = __builtin_fmaf(dx, (float)SI[v], -(dmx * M[v]));
+        lds_barrier();
+        const int nr = min(NWV, nb - b0);
+#pragma unroll
+        for (int e = 0; e < EPT; e++) {
+            const int u = min(tid + e * NTH, 1023), t = u >> 5;
+            for (int k = 0; k < nr; k++)
+                acc[e] = __builtin_fmaf(sD[k][t], reinterpret_cast<const float*>(sX[k])[t * kKqwTermRow + (u & 31)], acc[e]);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < EPT; e++) {
+        const int u = tid + e * NTH, t = tok0 + (u >> 5), row = row0 + (u & 31);
+        if (u < 1024 && t < m && row < d) out[(size_t)t * d + row] = acc[e];
+    }
+}
+
+// Waves over K of mm_batch_kq8w_kernel, or 0 where mm_batch_kq8_kernel is faster:
+// while a CU has at most three workgroups of 32 rows x 32 tokens (five of the
+// eight-wave ones, two of which it holds at once), and more than one block.  us,
+// here against there:
+//   10240 x 2560: 8 tokens (320 workgroups) 11.9 / 20.5, 37 (640) 17.3 / 21.1, 130
+//     (1600) 36.5 / 26.2
+//   2048 x 2560: 37 tokens (128) 6.4 / 16.5, 200 (448) 10.8 / 16.2, 511 (1024) 21.2 /
+//     17.3;  256 x 2560, 511 tokens (128) 6.6 / 16.0
+//   2560 x 2048: 37 tokens (160) 5.6 / 13.9, 511 (1280) 15.5 / 18.9
+//   2560 x 10240, 37 tokens (160, four rounds) 21.4 / 70.4;  2560 x 256, 37 tokens
+//     (one block) 4.9 / 4.5
+// The waves: all blocks in one round if ten can, else as few rounds as possible.
+int kq8w_waves(const int* d, int nseg, int m, int nb) {
+    if (nb < 2) return 0;
+    const int nwv = nb <= 2 ? 2 : nb <= 4 ? 4 : (nb + 7) / 8 <= (nb + 9) / 10 ? 8 : 10;
+    long long wgs = 0;
+    for (int k = 0; k < nseg; k++) wgs += (long long)((d[k] + 31) / 32) * ((m + 31) / 32);
+    return wgs <= (nb <= 8 ? 5LL : 3LL) * g4_num_cus() ? nwv : 0;
+}
+
+template <bool Q5, int NWV>
+void launch_mm_batch8w(const KqSegs& sg, const uint8_t* q8, int nb, int m) {
+    hipLaunchKernelGGL((mm_batch_kq8w_kernel<Q5, NWV>), dim3(sg.g0[sg.n] * ((m + 31) / 32)), dim3(64 * NWV), 0, g4_stream(),
+                       sg, q8, nb, m);
+}
+
 // ---- Q4_K / Q5_K through fp16 weight images (mm_batch_img_kernel) --------
 // The in-register weight decode of a quantized-tensor kernel (nibbles, Q5_K
 // high bits, the scales) is most of its vector instructions and sets its
@@ -1112,7 +1291,8 @@ extern "C" int g4_mm_batch_q8_multi(float* const* o, const void* const* w, const
         G4_CHECK_ARG(al16(o[k]) && al16(w[k]), "g4_mm_batch_q8: o and w must be 16-byte aligned");
         G4_CHECK_ARG(d[k] > 0 && (size_t)d[k] * nb * 176 < (1u << 31), "g4_mm_batch_q8: d=%d", d[k]);
     }
-    const int nwv = kq_waves(d, nseg, m), rg = 32 * nwv;   // rows per workgroup
+    const int kw = kq8w_waves(d, nseg, m, nb);             // waves over K, or 0
+    const int nwv = kw ? 1 : kq_waves(d, nseg, m), rg = 32 * nwv;   // rows per workgroup
     KqSegs sg{};
     sg.n = nseg;
     long long gx = 0;
@@ -1125,6 +1305,17 @@ extern "C" int g4_mm_batch_q8_multi(float* const* o, const void* const* w, const
     }
     sg.g0[nseg] = (int)gx;
     G4_CHECK_ARG(gx * ((m + 32 * kKqNT - 1) / (32 * kKqNT)) < (1LL << 31), "g4_mm_batch_q8: %d tokens too many", m);
+    if (kw) {
+        const uint8_t* q = (const uint8_t*)q8;
+        const bool q5 = type == G4_Q5_K;
+        switch (kw) {
+        case 2: q5 ? launch_mm_batch8w<true, 2>(sg, q, nb, m) : launch_mm_batch8w<false, 2>(sg, q, nb, m); break;
+        case 4: q5 ? launch_mm_batch8w<true, 4>(sg, q, nb, m) : launch_mm_batch8w<false, 4>(sg, q, nb, m); break;
+        case 8: q5 ? launch_mm_batch8w<true, 8>(sg, q, nb, m) : launch_mm_batch8w<false, 8>(sg, q, nb, m); break;
+        default: q5 ? launch_mm_batch8w<true, 10>(sg, q, nb, m) : launch_mm_batch8w<false, 10>(sg, q, nb, m); break;
+        }
+        return g4_check_launch("mm_batch_kq8w_kernel");
+    }
     if (type == G4_Q4_K) {
         if (nwv == 5) launch_mm_batch8<false, kKqNT, 5>(sg, (const uint8_t*)q8, nb, m);
         else launch_mm_batch8<false, kKqNT, 4>(sg, (const uint8_t*)q8, nb, m);

@@ -200,6 +200,26 @@ def test_mm_batch_q8_blocks_fold(lib, qtype, d, m):
 
 
 @pytest.mark.parametrize("qtype", [12, 13])
+@pytest.mark.parametrize("nb,d,m", [(2, 33, 1), (3, 31, 33), (4, 64, 32), (7, 96, 40), (8, 1000, 65), (9, 40, 5),
+                                    (10, 257, 64), (10, 1024, 31), (16, 70, 37), (21, 32, 95)])
+def test_mm_batch_q8_waves_over_k(lib, qtype, nb, d, m):
+    """The small grids, whose workgroups' waves take one block each (one round
+    of blocks or several, rows and tokens that end inside a tile): the bits of
+    the per-block terms folded in block order by the other kernel."""
+    from g4 import DBuf, upload_quant
+    n = 256 * nb
+    rng = np.random.default_rng(nb * 1000 + d + m + qtype)
+    w = upload_quant(lib, synth.rand_kquant(rng, qtype, d, n), qtype, n, d)
+    xd = DBuf.from_array(lib, _acts(rng, m, n))
+    q8, _ = _q8rows(lib, xd, n, m)
+    got = _mm_q8(lib, w, q8.ptr, n, d, m, qtype)
+    u, out = DBuf(lib, 4 * nb * m * d), DBuf(lib, 4 * m * d)
+    lib.g4_mm_batch_q8_blocks(u.ptr, w.ptr, q8.ptr, n, d, m, qtype)
+    lib.g4_fold_gelu_mul_q8(u.ptr, q8.ptr, n, None, 0, out.ptr, None, d, m)
+    assert np.array_equal(got.view(np.uint32), out.to_array(np.float32).reshape(m, d).view(np.uint32))
+
+
+@pytest.mark.parametrize("qtype", [12, 13])
 def test_mm_batch_q8_multi(lib, orc, qtype):
     """Three matrices of one type over the same Q8_K rows in one launch (the
     engine's Q|K and gate|up): each output equals the single-matrix launch
