@@ -1604,21 +1604,9 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
 // issue (half of the time) and the matrix cores (a quarter), which a wave
 // overlaps only in part.
 constexpr int kR5Keys = 32, kR5KRow = 2080;
-typedef float f2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(1))) const f2_t g4_gf2_t;
-typedef _Float16 ah2_t __attribute__((ext_vector_type(2)));
+typedef h2v_t ah2_t;
 
-// x sf and y sf as fp16 hi + lo (round to nearest; x sf - hi is exact)
-__device__ __forceinline__ void split2(float x, float y, float sf, ah2_t& hi, ah2_t& lo) {
-    hi = __builtin_convertvector((f2_t{x * sf, y * sf}), ah2_t);
-    lo = __builtin_convertvector((f2_t{__builtin_fmaf(x, sf, -(float)hi[0]), __builtin_fmaf(y, sf, -(float)hi[1])}), ah2_t);
-}
-// max(|x|, |y|, m) in one instruction (fmaxf on loaded values is three)
-__device__ __forceinline__ float max3_abs(float x, float y, float m) {
-    float r;
-    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(x), "v"(y), "v"(m));
-    return r;
-}
 // e^x for x <= kRowsLazy, 0 below the smallest normal number: 2^(x log2 e) with
 // the product's rounding error put back to first order (within 2 ulp)
 __device__ __forceinline__ float exp_le(float x) {

@@ -66,6 +66,15 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // lgkmcnt left at their maxima, i.e. not waited for)
 constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
+// 16 bytes per lane from a buffer straight into LDS at lds + 16 * lane (the
+// LDS address is wave-uniform: it goes to M0).  A plain device function: in
+// a kernel template's own body the builtin keeps the host pass from
+// emitting the kernel's launch stub.
+typedef __attribute__((address_space(3))) void lds_void;
+__device__ __forceinline__ void buf_load_lds16(__amdgpu_buffer_rsrc_t r, uint8_t* lds, int voff, int soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, soff, 0, 0);
+}
+
 bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace

@@ -991,15 +991,6 @@ __global__ __launch_bounds__(256) void gelu_mul_split_kernel(const float* __rest
 // row 16 rt + i.
 constexpr int kXsStride = kSplitBlk + 32;   // LDS bytes per staged token
 
-// 16 bytes per lane from a buffer straight into LDS at lds + 16 * lane (the
-// LDS address is wave-uniform: it goes to M0).  A plain device function: in
-// a kernel template's own body the builtin keeps the host pass from
-// emitting the kernel's launch stub.
-typedef __attribute__((address_space(3))) void lds_void;
-__device__ __forceinline__ void buf_load_lds16(__amdgpu_buffer_rsrc_t r, uint8_t* lds, int voff, int soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, soff, 0, 0);
-}
-
 // SP (two stages only): the next block's copies are issued one per product
 // step of this block instead of all at its start, and one barrier per block
 // suffices

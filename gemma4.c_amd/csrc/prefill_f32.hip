@@ -17,11 +17,10 @@
 // Work split.  The four waves of a workgroup share one output tile and split
 // K: wave w takes the Q6_K blocks b = w (mod 4), or of every 256 bf16
 // elements those from 64 w, and the four partial tiles are added through LDS
-// at the end, (a0 + a1) + (a2 + a3).  A wave thus loads each operand once,
-// straight into the registers it feeds the matrix cores from (no staging, no
-// barrier in the loop), and splits each activation and decodes each weight
-// once per workgroup.  The order of a token's sums depends on n alone, so
-// every tile shape gives the same bits.
+// at the end, (a0 + a1) + (a2 + a3).  A wave thus needs each operand once, reads
+// nothing that another wave brought (no barrier in the loop), and splits each
+// activation and decodes each weight once per workgroup.  The order of a token's
+// sums depends on n alone, so every tile shape gives the same bits.
 #include "g4_device.h"
 #include "g4_internal.h"
 #include "g4_tile.h"
@@ -75,53 +74,70 @@ __device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, flo
 }
 
 // ---- bf16 weights ---------------------------------------------------------
+// Activations come by copies of whole lines (below: mm_batch_q6_kernel), a unit of
+// 64 elements (two lines a token) ahead; weight rows straight into registers.
+// Line (s, token): chunk c of 16 bytes in slot c ^ bf_swz(token).
+__device__ __forceinline__ int bf_swz(int t) { return ((t >> 1) & 1) | ((t >> 1) & 4); }
+
 template <int NT, int RT>
 __global__ __launch_bounds__(256) void mm_batch_bf16_kernel(const uint16_t* __restrict__ w, const float* __restrict__ x,
                                                             float* __restrict__ out, int n, int d, int m, int vec) {
-    __shared__ f4_t red[4 * red_tiles(NT * RT) * 64];
+    constexpr int kUnit = 4096 * NT;      // bytes of a unit of the tile's tokens
+    constexpr size_t kRed = sizeof(f4_t) * 4 * red_tiles(NT * RT) * 64, kStages = (size_t)4 * 2 * kUnit;
+    __shared__ __align__(16) uint8_t lds[kStages > kRed ? kStages : kRed];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, g = lane >> 4;
     int bx, by;
     xcd_tile((m + 16 * NT - 1) / (16 * NT), bx, by);
     const int row0 = bx * 16 * RT, tok0 = by * 16 * NT;
     const int nb = n >> 8;
-    // of the wave's 64 elements of a block, lane group g takes 16 g .. + 15 and
-    // step s of the two 16 g + 8 s .. + 7
-    const float* px[NT];
-    const uint16_t* pw[RT];
+    uint8_t* stages = lds + (size_t)wave * 2 * kUnit;
+    uint32_t vx[NT][2], vw[RT];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) px[nt] = x + (size_t)min(tok0 + 16 * nt + i, m - 1) * n + 64 * wave + 8 * g;
+    for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) pw[rt] = w + (size_t)min(row0 + 16 * rt + i, d - 1) * n + 64 * wave + 8 * g;
-
-    struct Ops {
-        uint4 x[NT][4];
-        uint4 w[RT][2];
-    };
-    auto load = [&](int b, Ops& r) {
-        const size_t o = (size_t)b * 256;
+        for (int q = 0; q < 2; q++) {
+            const int t = 8 * q + (lane >> 3);
+            vx[nt][q] = (uint32_t)(min(tok0 + 16 * nt + t, m - 1) - tok0) * (uint32_t)n * 4u +
+                        16u * (uint32_t)((lane & 7) ^ bf_swz(t));
+        }
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) vw[rt] = (uint32_t)(min(row0 + 16 * rt + i, d - 1) - row0) * (uint32_t)n * 2u + 16u * g;
+    // of the wave's 64 elements of a block, step s of two takes 32 s .. + 31, lane
+    // group g 8 of them.  (The block's address goes into the descriptors: offsets
+    // stay within a tile's rows.)
+    uint4 W[2][RT][2];
+    auto load = [&](int b, int st) {
+        const size_t o = (size_t)b * 256 + 64 * wave;
+        const __amdgpu_buffer_rsrc_t rx =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(x + (size_t)tok0 * n + o), (short)0, -1, kBufWord3);
+        const __amdgpu_buffer_rsrc_t rw =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)row0 * n + o), (short)0, -1, kBufWord3);
 #pragma unroll
         for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-            for (int k = 0; k < 4; k++) r.x[nt][k] = reinterpret_cast<const uint4*>(px[nt] + o + 32 * (k >> 1))[k & 1];
+            for (int q = 0; q < 4; q++)   // lines 8 q .. 8 q + 7: step q / 2, tokens 8 (q & 1) ..
+                buf_load_lds16(rx, stages + st * kUnit + nt * 4096 + q * 1024, (int)vx[nt][q & 1], 128 * (q >> 1));
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-            for (int k = 0; k < 2; k++) r.w[rt][k] = *reinterpret_cast<const uint4*>(pw[rt] + o + 32 * k);
+            for (int k = 0; k < 2; k++) W[st][rt][k] = buf_load16(rw, (int)vw[rt], 64 * k);
     };
     f4_t acc[RT][NT];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) acc[rt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
-    auto compute = [&](const Ops& r) {
+    auto compute = [&](int st) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             b8_t xt[3][NT];
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
-                uint32_t f[8] = {r.x[nt][2 * s].x,     r.x[nt][2 * s].y,     r.x[nt][2 * s].z,     r.x[nt][2 * s].w,
-                                 r.x[nt][2 * s + 1].x, r.x[nt][2 * s + 1].y, r.x[nt][2 * s + 1].z, r.x[nt][2 * s + 1].w};
+                const uint8_t* line = stages + st * kUnit + nt * 4096 + (16 * s + i) * 128;
+                const uint4 f0 = *reinterpret_cast<const uint4*>(line + 16 * ((2 * g) ^ bf_swz(i)));
+                const uint4 f1 = *reinterpret_cast<const uint4*>(line + 16 * ((2 * g + 1) ^ bf_swz(i)));
+                uint32_t f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
 #pragma unroll
                 for (int t = 0; t < 3; t++) {
                     uint32_t p[4];
@@ -136,7 +152,7 @@ __global__ __launch_bounds__(256) void mm_batch_bf16_kernel(const uint16_t* __re
             }
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
-                const b8_t a = __builtin_bit_cast(b8_t, r.w[rt][s]);
+                const b8_t a = __builtin_bit_cast(b8_t, W[st][rt][s]);
 #pragma unroll
                 for (int t = 2; t >= 0; t--)
 #pragma unroll
@@ -145,19 +161,23 @@ __global__ __launch_bounds__(256) void mm_batch_bf16_kernel(const uint16_t* __re
             }
         }
     };
-    // the next block's operands load while the current one's are multiplied
-    // (past the end the last block again: no branch around the loads)
-    Ops r0, r1;
-    load(0, r0);
-    int b = 0;
-    for (; b + 1 < nb; b += 2) {
-        load(b + 1, r1);
-        compute(r0);
-        load(min(b + 2, nb - 1), r0);
-        compute(r1);
+    // a block's operands, sent a block ago, have landed; the next one's are sent
+    // while it is multiplied (past the end the last block again, read by nobody)
+    auto block = [&](int b, int st) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        asm volatile("" ::: "memory");
+        load(min(b + 1, nb - 1), st ^ 1);
+        compute(st);
+    };
+    load(0, 0);
+    for (int b = 0; b < nb; b += 2) {
+        block(b, 0);
+        if (b + 1 < nb) block(b + 1, 1);
     }
-    if (b < nb) compute(r0);
-
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the last copies land before the sums take their place
+    __syncthreads();
+    f4_t* red = reinterpret_cast<f4_t*>(lds);
     reduce_store<NT, RT>(acc, red, out, row0, tok0, d, m, vec, [&](int tok, int row) {
         float sum = 0.0f;
         for (int k = 0; k < n; k++)
@@ -277,10 +297,23 @@ __global__ __launch_bounds__(64 * RW) void mm_batch_f32_kernel(const uint16_t* _
 }
 
 // ---- Q6_K weights -----------------------------------------------------------
-template <int NT, int RT>
+// The activations come by global -> LDS copies of whole 128-byte lines, eight
+// lines an instruction: an instruction costs the L1 four cycles for every line
+// it touches, and loads straight into operand order (a 16-byte piece of 32 lines)
+// had it busy the whole time.  Each wave copies its own groups, NS - 1 of them
+// ahead (a group: the 64 elements a token of one scale, two 128-byte lines), and
+// no other wave reads them, so there is no barrier in the loop.  Line (h, token):
+// chunk c of 16 bytes lies in slot c ^ line_swz(token), which spreads the sixteen
+// lanes that LDS serves at once over all banks.
+__device__ __forceinline__ int line_swz(int t) { return ((t >> 1) & 1) | ((t >> 2) & 2); }
+
+template <int NT, int RT, int NS>
 __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                           float* __restrict__ out, int n, int d, int m, int vec) {
-    __shared__ f4_t red[4 * red_tiles(NT * RT) * 64];
+    static_assert(NS == 2 || NS == 4, "a block's four groups use the stages in turn");
+    constexpr int kGroup = 4096 * NT;     // bytes of a group of the tile's tokens
+    constexpr size_t kRed = sizeof(f4_t) * 4 * red_tiles(NT * RT) * 64, kStages = (size_t)4 * NS * kGroup;
+    __shared__ __align__(16) uint8_t lds[kStages > kRed ? kStages : kRed];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, g = lane >> 4, h = g >> 1, s = g & 1;
     int bx, by;
@@ -290,45 +323,53 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
     const size_t nblk = (size_t)d * nb;
     const Q6KPlanes P = q6k_planes(nblk);
 
+    // copy q of a group and 16-token tile: lines 8 q .. 8 q + 7, line l is half
+    // l / 16 of token l % 16
+    uint8_t* stages = lds + (size_t)wave * NS * kGroup;
+    uint32_t vx[NT][2];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int t = 8 * q + (lane >> 3);
+            vx[nt][q] = (uint32_t)(min(tok0 + 16 * nt + t, m - 1) - tok0) * (uint32_t)n * 4u +
+                        16u * (uint32_t)((lane & 7) ^ line_swz(t));
+        }
+    auto copy_x = [&](int b, int k, int st) {
+        // (the block's address goes into the descriptor: offsets stay within a tile's rows)
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(x + (size_t)tok0 * n + (size_t)b * 256 + 32 * k), (short)0, -1, kBufWord3);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                buf_load_lds16(rx, stages + st * kGroup + nt * 4096 + q * 1024, (int)vx[nt][q & 1], 512 * (q >> 1));
+    };
+
     // lane group g's elements of a block: 128 h + 32 k + 16 s + 8 half + t, in
     // step c = 2 k + half (layout.hip); group k of two steps is 16 in a row
-    const float* px[NT];
+    uint32_t rB[RT];                      // first block of the row, from the tile's first row's
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) px[nt] = x + (size_t)min(tok0 + 16 * nt + i, m - 1) * n + 128 * h + 16 * s;
-    size_t rB[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++) rB[rt] = (size_t)min(row0 + 16 * rt + i, d - 1) * nb;
-    const uint8_t* wql = w + P.ql + 32 * g;
-    const uint8_t* wqh = w + P.qh + 16 * g;
-    const uint8_t* wsc = w + P.sc + 8 * h;
-    const uint8_t* wd = w + P.d;
-
+    for (int rt = 0; rt < RT; rt++) rB[rt] = (uint32_t)(min(row0 + 16 * rt + i, d - 1) - row0) * (uint32_t)nb;
+    const size_t b0 = (size_t)row0 * nb;
+    auto rsrc = [&](size_t off) { return __builtin_amdgcn_make_buffer_rsrc((void*)(w + off), (short)0, -1, kBufWord3); };
+    const __amdgpu_buffer_rsrc_t rql = rsrc(P.ql + b0 * 128), rqh = rsrc(P.qh + b0 * 64), rsc = rsrc(P.sc + b0 * 16),
+                                 rd = rsrc(P.d + b0 * 2);
     struct WRaw {
         uint4 ql[RT][2];
         uint4 qh[RT];
         uint2 sc[RT];
         uint32_t dh[RT];
     };
-    struct XRaw {
-        f4_t v[NT][4];
-    };
     auto load_w = [&](int b, WRaw& r) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
-            const size_t blk = rB[rt] + b;
-            r.ql[rt][0] = reinterpret_cast<const uint4*>(wql + blk * 128)[0];
-            r.ql[rt][1] = reinterpret_cast<const uint4*>(wql + blk * 128)[1];
-            r.qh[rt] = *reinterpret_cast<const uint4*>(wqh + blk * 64);
-            r.sc[rt] = *reinterpret_cast<const uint2*>(wsc + blk * 16);
-            r.dh[rt] = *reinterpret_cast<const uint16_t*>(wd + blk * 2);
+            r.ql[rt][0] = buf_load16(rql, (int)(rB[rt] * 128 + 32 * g), b * 128);
+            r.ql[rt][1] = buf_load16(rql, (int)(rB[rt] * 128 + 32 * g + 16), b * 128);
+            r.qh[rt] = buf_load16(rqh, (int)(rB[rt] * 64 + 16 * g), b * 64);
+            r.sc[rt] = buf_load8(rsc, (int)(rB[rt] * 16 + 8 * h), b * 16);
+            r.dh[rt] = __builtin_amdgcn_raw_buffer_load_b16(rd, (int)(rB[rt] * 2), b * 2, 0);
         }
-    };
-    auto load_x = [&](int b, int k, XRaw& r) {
-        const size_t o = (size_t)b * 256 + 32 * k;
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) r.v[nt][q] = reinterpret_cast<const f4_t*>(px[nt] + o)[q];
     };
 
     f4_t acc[RT][NT];
@@ -338,17 +379,19 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
         for (int nt = 0; nt < NT; nt++) acc[rt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
     const h2_t m1056 = {(_Float16)-1056.0f, (_Float16)-1056.0f};
 
-    auto group = [&](const XRaw& r, int k, const WRaw& wc, const float (&dw)[RT][4]) {
+    auto group = [&](int st, int k, const WRaw& wc, const float (&dw)[RT][4]) {
         h8_t Xh[2][NT], Xl[2][NT];
         float ts[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            float f[16];
-#pragma unroll
-            for (int q = 0; q < 16; q++) f[q] = r.v[nt][q >> 2][q & 3];
+            f4_t f[4];
             float mx = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 16; q++) mx = fmaxf(mx, fabsf(f[q]));
+            for (int q = 0; q < 4; q++) {
+                f[q] = *reinterpret_cast<const f4_t*>(stages + st * kGroup + nt * 4096 + (16 * h + i) * 128 +
+                                                      16 * ((4 * s + q) ^ line_swz(i)));
+                mx = max3_abs(f[q][2], f[q][3], max3_abs(f[q][0], f[q][1], mx));
+            }
             // the largest of the token's 64 (lanes i, i + 16, i + 32, i + 48)
             const uint32_t u = __float_as_uint(mx);
             const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
@@ -359,14 +402,14 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
             const float sf = __uint_as_float((uint32_t)fe << 23);
             ts[nt] = __uint_as_float((uint32_t)(254 - fe) << 23);
 #pragma unroll
-            for (int st = 0; st < 2; st++)
+            for (int st2 = 0; st2 < 2; st2++) {
+                h2v_t hi[4], lo[4];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float v = f[8 * st + j] * sf;
-                    const _Float16 hv = (_Float16)v;
-                    Xh[st][nt][j] = hv;
-                    Xl[st][nt][j] = (_Float16)(v - (float)hv);
-                }
+                for (int q = 0; q < 4; q++)
+                    split2(f[2 * st2 + (q >> 1)][2 * (q & 1)], f[2 * st2 + (q >> 1)][2 * (q & 1) + 1], sf, hi[q], lo[q]);
+                Xh[st2][nt] = __builtin_bit_cast(h8_t, make_uint4(h2_bits(hi[0]), h2_bits(hi[1]), h2_bits(hi[2]), h2_bits(hi[3])));
+                Xl[st2][nt] = __builtin_bit_cast(h8_t, make_uint4(h2_bits(lo[0]), h2_bits(lo[1]), h2_bits(lo[2]), h2_bits(lo[3])));
+            }
         }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
@@ -407,10 +450,8 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
                     acc[rt][nt][v] = __builtin_fmaf(S[nt][v] * ts[nt], dw[rt][v], acc[rt][nt][v]);
         }
     };
-    XRaw x0, x1;
     auto block = [&](int b, const WRaw& wc, WRaw& wn) {
         const int bn = b + 4 < nb ? b + 4 : b;   // (the last block again at the end: no branch around the loads)
-        load_w(bn, wn);
         float dw[RT][4];                         // d of rows 4 g + v
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
@@ -418,24 +459,34 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
 #pragma unroll
             for (int v = 0; v < 4; v++) dw[rt][v] = __shfl(dl, 4 * g + v, 64);
         }
-        load_x(b, 1, x1);
-        group(x0, 0, wc, dw);
-        load_x(b, 2, x0);
-        group(x1, 1, wc, dw);
-        load_x(b, 3, x1);
-        group(x0, 2, wc, dw);
-        load_x(bn, 0, x0);
-        group(x1, 3, wc, dw);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            // this group's copies have landed: at most the ones of the NS - 2
+            // groups after it are in flight (weight loads among them only make
+            // the wait longer), and the group before it has been read
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(4 * NT * (NS - 2)));
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);   // (a group's operands are not formed ahead of it)
+            constexpr int kAhead = NS - 1;
+            copy_x(k + kAhead < 4 ? b : bn, (k + kAhead) & 3, (k + kAhead) & (NS - 1));
+            if (k == 0) load_w(bn, wn);
+            group(k & (NS - 1), k, wc, dw);
+        }
     };
     if (wave < nb) {
         WRaw w0, w1;
         load_w(wave, w0);
-        load_x(wave, 0, x0);
+#pragma unroll
+        for (int k = 0; k < NS - 1; k++) copy_x(wave, k, k);
         for (int b = wave; b < nb; b += 8) {
             block(b, w0, w1);
             if (b + 4 < nb) block(b + 4, w1, w0);
         }
     }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the last copies, read by nobody, land before the sums go there
+    __syncthreads();
+    f4_t* red = reinterpret_cast<f4_t*>(lds);
     reduce_store<NT, RT>(acc, red, out, row0, tok0, d, m, vec, [&](int tok, int row) {
         float sum = 0.0f;
         for (int k = 0; k < n; k++)
@@ -444,19 +495,18 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
     });
 }
 
-// Tile shapes.  A tile's time does not depend on how many other workgroups
-// share the chip until a CU holds a second one, so a launch takes
-// ceil(workgroups / CUs) times the tile's own cost; the table's costs are the
-// times of one round in us (MI355X; bf16 over 2560 columns, where they follow
-// the bytes a tile loads, 2 NT + RT; Q6_K over 10240).  The cheapest shape is
-// taken; small batches get small tiles and so more workgroups.
-//   bf16 10752 x 2560, 512 tokens: 64 x 128 tiles 155 us, 64 x 64 198, 32 x 64
-//     223; 130 tokens 52 / 66 / 77; 37 tokens 52 / 32 / 41; 6 tokens 16 x 32
-//     17.6, 64 x 64 27.  fp32 matrix cores (64 x 32 tiles) before: 307, 106,
-//     55, 42.
-//   Q6_K 2560 x 10240, 512 tokens: 32 x 80 tiles 167 us, 16 x 16 498; 37
-//     tokens 16 x 32 38, 32 x 80 81; 6 tokens 16 x 16 23, 16 x 32 33.  fp32
-//     matrix cores before: 344, 94, 92.
+// Tile shapes.  A launch takes about ceil(workgroups / CUs) times its tile's cost;
+// the table's costs are the times of one round in us (MI355X; bf16 over 2560
+// columns, Q6_K over 10240) and the cheapest shape is taken, so small batches get
+// small tiles and more workgroups.  us, and in brackets the same tiles with every
+// load straight into operand order, and the fp32 matrix cores before:
+//   bf16 10752 x 2560, 512 tokens: 64 x 128 tiles 133 (155, 307), 64 x 64 167; 130
+//     tokens 45 (52, 106); 37 tokens, 64 x 64 28 (32, 55); 6 tokens, 16 x 16 17 (18, 42)
+//   Q6_K 2560 x 10240, 512 tokens: 32 x 80 tiles 164 (167, 344), 16 x 16 454; 130
+//     tokens, 32 x 64 65 (71, 139); 37 tokens, 16 x 32 32 (38, 94); 6 tokens, 16 x 16
+//     23 (23, 92)
+// The large Q6_K tile holds 460 registers: one wave a SIMD, whose splits, decode
+// and products overlap only in part (64 x 80 tiles spill: 216 us and more).
 struct Tile {
     int nt, rt, cost;
     void (*launch)(const void* w, const float* x, float* o, int n, int d, int m);
@@ -468,20 +518,20 @@ void launch_bf16(const void* w, const float* x, float* o, int n, int d, int m) {
     hipLaunchKernelGGL((mm_batch_bf16_kernel<NT, RT>), dim3(gx * gy), dim3(256), 0, g4_stream(), (const uint16_t*)w, x, o, n,
                        d, m, (int)(d % 4 == 0 && al16(o)));
 }
-template <int NT, int RT>
+template <int NT, int RT, int NS>
 void launch_q6(const void* w, const float* x, float* o, int n, int d, int m) {
     const int gx = (d + 16 * RT - 1) / (16 * RT), gy = (m + 16 * NT - 1) / (16 * NT);
-    hipLaunchKernelGGL((mm_batch_q6_kernel<NT, RT>), dim3(gx * gy), dim3(256), 0, g4_stream(), (const uint8_t*)w, x, o, n, d,
+    hipLaunchKernelGGL((mm_batch_q6_kernel<NT, RT, NS>), dim3(gx * gy), dim3(256), 0, g4_stream(), (const uint8_t*)w, x, o, n, d,
                        m, (int)(d % 4 == 0 && al16(o)));
 }
 
-const Tile kTilesBf16[] = {{1, 1, 3, launch_bf16<1, 1>},  {1, 2, 4, launch_bf16<1, 2>},  {2, 4, 8, launch_bf16<2, 4>},
-                           {4, 4, 12, launch_bf16<4, 4>}, {4, 6, 14, launch_bf16<4, 6>}, {4, 8, 16, launch_bf16<4, 8>}};
-const Tile kTilesQ6[] = {{1, 1, 25, launch_q6<1, 1>},
-                         {1, 2, 32, launch_q6<1, 2>},
-                         {2, 2, 52, launch_q6<2, 2>},
-                         {2, 4, 71, launch_q6<2, 4>},
-                         {2, 5, 81, launch_q6<2, 5>}};
+const Tile kTilesBf16[] = {{1, 1, 5, launch_bf16<1, 1>},  {1, 2, 8, launch_bf16<1, 2>},  {2, 4, 16, launch_bf16<2, 4>},
+                           {4, 4, 28, launch_bf16<4, 4>}, {4, 6, 35, launch_bf16<4, 6>}, {4, 8, 44, launch_bf16<4, 8>}};
+const Tile kTilesQ6[] = {{1, 1, 20, launch_q6<1, 1, 4>},
+                         {1, 2, 27, launch_q6<1, 2, 4>},
+                         {2, 2, 43, launch_q6<2, 2, 4>},
+                         {2, 4, 65, launch_q6<2, 4, 4>},
+                         {2, 5, 81, launch_q6<2, 5, 4>}};
 
 template <int N>
 const Tile& pick_tile(const Tile (&tiles)[N], int d, int m) {
@@ -514,7 +564,17 @@ extern "C" int g4_mm_batch_bf16_f32(float* o, const float* x, const void* w, int
 }
 
 int g4_mm_batch_f32(float* o, const float* x, const void* w, int n, int d, int m, int type) {
-    const Tile& t = type == G4_BF16 ? pick_tile(kTilesBf16, d, m) : pick_tile(kTilesQ6, d, m);
-    t.launch(w, x, o, n, d, m);
+    if (n < 1 << 24) {
+        const Tile& t = type == G4_BF16 ? pick_tile(kTilesBf16, d, m) : pick_tile(kTilesQ6, d, m);
+        t.launch(w, x, o, n, d, m);
+    } else {
+        // a tile's rows must lie within 32-bit offsets: one token (and bf16 row) a launch
+        for (int t = 0; t < m; t++)
+            for (int r = 0; r < (type == G4_BF16 ? d : 1); r++) {
+                const float* xt = x + (size_t)t * n;
+                if (type == G4_BF16) launch_bf16<1, 1>((const uint16_t*)w + (size_t)r * n, xt, o + (size_t)t * d + r, n, 1, 1);
+                else launch_q6<1, 1, 4>(w, xt, o + (size_t)t * d, n, d, 1);
+            }
+    }
     return g4_check_launch(type == G4_BF16 ? "mm_batch_bf16_kernel" : "mm_batch_q6_kernel");
 }
