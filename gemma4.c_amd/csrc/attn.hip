@@ -1946,6 +1946,9 @@ void launch_merge(const AttnArgs& a, const dim3& grid) {
 // layer, where another order of sums moves some code by one and the model carries
 // it on, so it keeps the bits, and the tokens, it had.
 constexpr int kRowsQ8Keys = 1024;
+// up to 23 keys the 16-key tiles are faster (11 rows at 0: 19.2 / 18.0, 17: 21.6 /
+// 20.1, 24: 21.5 / 21.8)
+constexpr int kRowsFewKeys = 23;
 
 int launch_attn(const AttnArgs& a) {
     const int kvm = a.n_heads / a.n_kv;
@@ -1960,7 +1963,7 @@ int launch_attn(const AttnArgs& a) {
             hipLaunchKernelGGL(attn_rows_h16_kernel<256>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
             launch_merge<256>(a, dim3(a.n_heads, 1, zq));
         } else {
-            if (!a.q8 || a.p0 + a.qrows > kRowsQ8Keys) hipLaunchKernelGGL(attn_rows512_kernel, rgrid, dim3(512), 0, g4_stream(), a);
+            if (a.p0 + a.qrows > (a.q8 ? kRowsQ8Keys : kRowsFewKeys)) hipLaunchKernelGGL(attn_rows512_kernel, rgrid, dim3(512), 0, g4_stream(), a);
             else hipLaunchKernelGGL(attn_rows_mfma_kernel<512>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
             launch_merge<512>(a, dim3(a.n_heads, 2, zq));
         }

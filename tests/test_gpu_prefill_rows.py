@@ -353,6 +353,8 @@ def test_attn_decode_rows_peaked_small(lib, orc, hd):
 ROWS512_CASES = [
     # p0, m, G, window, ring, scale of K, scale of V
     (0, 1, 1, 0, 0, 1.0, 1.0),             # a single row and key
+    (0, 23, 2, 0, 0, 1.0, 1.0),            # the last size of the fp32 kernel, and the next
+    (0, 24, 2, 0, 0, 1.0, 1.0),
     (0, 37, 3, 0, 0, 1.0, 1.0),            # rows that end inside a 16-row block, chunks inside a tile
     (995, 61, 16, 0, 0, 1.0, 1.0),         # cache and chunk rows in one tile, chunks of whole tiles
     (700, 50, 4, 300, 300, 1.0, 1.0),      # a wrapped ring, windows that start inside a tile
