@@ -1401,22 +1401,41 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
 typedef _Float16 ah4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 ah8_t __attribute__((ext_vector_type(8)));
 
+typedef __attribute__((address_space(1))) const f2_t g4_gf2_t;
+typedef h2v_t ah2_t;
+__device__ __forceinline__ ah4_t join4(ah2_t a, ah2_t b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3); }
+
+// the largest over lanes j, j + 16, j + 32, j + 48
+__device__ __forceinline__ float groups_max(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t w = __float_as_uint(fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1])));
+    const auto q = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
 __device__ __forceinline__ _Float16 split_hi(float v) { return (_Float16)v; }
 __device__ __forceinline__ _Float16 split_lo(float v, _Float16 h) { return (_Float16)(v - (float)h); }
 
+// Two barriers a tile, waiting for LDS only: wave w stages keys 4w .. 4w + 3 whole
+// (addresses by selects: a load behind a branch waits for all before it), V
+// between the score products, the next tile's K between the output products;
+// operands are read ahead of their products.  LDS: K rows of 544 bytes, V
+// transposed in rows of four 8-byte slots, slot g at g ^ 2 (dim / 8 & 1): both
+// read without bank conflicts.  511 rows at position 1001, window 512, four
+// chunks, with the merge: 42.4 us with per-lane addresses behind branches, full
+// barriers and one fp16 a store for V, 35.7 now (same bits); 16 rows over 116
+// keys 28.9 and 22.6.  About 2 us a tile, a chain of latencies on one wave a SIMD.
 template <int HD>
-__global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(HD == 256 ? 2 : 1))) void attn_rows_h16_kernel(AttnArgs a) {
-    constexpr int NTH = 64 * kRowsKVM;
-    constexpr int KS = HD + 8;            // K row stride (fp16)
-    constexpr int VS = 16 + 4;            // V^T row stride (fp16): 16 keys + pad
+__global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(2))) void attn_rows_h16_kernel(AttnArgs a) {
+    static_assert(HD == 256, "the staging of a wave: one float4 of K, two float2 of V a lane and key");
+    constexpr int KS = HD + 16;           // K row stride (fp16)
     constexpr int NS = HD / 32;           // score steps
     constexpr int NB = HD / 16;           // O tiles
-    constexpr int LU = 16 * (HD / 4) / NTH;   // float4 of K (and of V) per thread and tile
-    static_assert(LU * NTH == 16 * (HD / 4), "tile staging");
     __shared__ __align__(16) _Float16 kh[16 * KS], kl[16 * KS];
-    __shared__ __align__(16) _Float16 vh[HD * VS], vl[HD * VS];
+    __shared__ __align__(16) _Float16 vh[HD * 16], vl[HD * 16];
     const int c = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, j = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, j = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int head = kvh * kRowsKVM + wave;
     const int M = a.qrows;
     const int z0 = 16 * rb, z1 = min(z0 + 16, M) - 1;
@@ -1428,26 +1447,49 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
     const int qp = a.p0 + z;
     const int qlo = a.window > 0 ? max(0, qp + 1 - a.window) : 0;
 
-    f4_t kr[LU], vr[LU];
-    const float* kcb = a.kc + (size_t)kvh * HD;
-    const float* vcb = a.vc + (size_t)kvh * HD;
-    const float* kqb = a.kchunk + (size_t)kvh * HD;
-    const float* vqb = a.vchunk + (size_t)kvh * HD;
+    // past the chunk the last position again (weight 0)
+    f4_t kr[4];
+    f2_t vr[4][2];
     const int tl = ce - 1;
-    auto load_tile = [&](int t0) {
+    const unsigned ring = a.ring > 0 ? (unsigned)a.ring : 0x7fffffffu;
+    auto row_of = [&](int t0, int r, const float* cache, const float* own) {
+        const int tf = min(t0 + 4 * wave, tl), t = min(t0 + 4 * wave + r, tl);
+        unsigned slot = (unsigned)tf % ring + (unsigned)(t - tf);
+        slot = slot >= ring ? slot - ring : slot;
+        const bool mine = t >= a.p0;
+        const size_t off = (size_t)(mine ? (unsigned)(t - a.p0) : slot) * a.kv_stride + (size_t)kvh * HD;
+        return (mine ? (uintptr_t)own : (uintptr_t)cache) + 4 * off;
+    };
+    auto load_k = [&](int t0) {
 #pragma unroll
-        for (int u = 0; u < LU; u++) {
-            const int idx = u * NTH + tid, key = idx / (HD / 4), c4 = idx - key * (HD / 4);
-            const int t = min(t0 + key, tl);
-            const bool own = t >= a.p0;
-            const size_t off = (size_t)(own ? t - a.p0 : attn_slot(a, t)) * a.kv_stride;
-            const uintptr_t kb = own ? (uintptr_t)kqb : (uintptr_t)kcb;
-            const uintptr_t vb = own ? (uintptr_t)vqb : (uintptr_t)vcb;
-            kr[u] = reinterpret_cast<const g4_gf4_t*>(kb + 4 * off)[c4];
-            vr[u] = reinterpret_cast<const g4_gf4_t*>(vb + 4 * off)[c4];
+        for (int r = 0; r < 4; r++) kr[r] = reinterpret_cast<const g4_gf4_t*>(row_of(t0, r, a.kc, a.kchunk))[lane];
+    };
+    auto load_v = [&](int t0) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uintptr_t p = row_of(t0, r, a.vc, a.vchunk);
+#pragma unroll
+            for (int k = 0; k < 2; k++) vr[r][k] = reinterpret_cast<const g4_gf2_t*>(p)[lane + 64 * k];
         }
     };
-    load_tile(cb);   // an empty chunk (cb > hi) loads position hi: ce - 1 = hi
+    auto stage_k = [&](int r) {
+        ah2_t h0, l0, h1, l1;
+        split2(kr[r][0], kr[r][1], 1.0f, h0, l0);
+        split2(kr[r][2], kr[r][3], 1.0f, h1, l1);
+        *reinterpret_cast<ah4_t*>(kh + (4 * wave + r) * KS + 4 * lane) = join4(h0, h1);
+        *reinterpret_cast<ah4_t*>(kl + (4 * wave + r) * KS + 4 * lane) = join4(l0, l1);
+    };
+    auto stage_v = [&](int k, int x) {
+        const int dim = 128 * k + 2 * lane + x, at = dim * 16 + 4 * (wave ^ (2 * ((lane >> 2) & 1)));
+        ah2_t h0, l0, h1, l1;
+        split2(vr[0][k][x], vr[1][k][x], 1.0f, h0, l0);
+        split2(vr[2][k][x], vr[3][k][x], 1.0f, h1, l1);
+        *reinterpret_cast<ah4_t*>(vh + at) = join4(h0, h1);
+        *reinterpret_cast<ah4_t*>(vl + at) = join4(l0, l1);
+    };
+    // (an empty chunk, cb > hi, loads position hi: ce - 1 = hi)
+    load_k(cb);
+    load_v(cb);
 
     ah8_t qh[NS], ql[NS];
     {
@@ -1465,49 +1507,44 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
             }
         }
     }
+    if (cb < ce) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) stage_k(r);
+        load_k(cb + 16);
+    }
 
     float m = -INFINITY, lsum = 0.0f;   // lsum: this lane's keys only (summed over the groups at the end)
     f4_t o[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) o[b] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
     for (int t0 = cb; t0 < ce; t0 += 16) {
-        __syncthreads();   // every wave is done with the previous tile
-#pragma unroll
-        for (int u = 0; u < LU; u++) {
-            const int idx = u * NTH + tid, key = idx / (HD / 4), c4 = idx - key * (HD / 4);
-            ah4_t h4, l4;
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                const _Float16 h = split_hi(kr[u][x]);
-                h4[x] = h;
-                l4[x] = split_lo(kr[u][x], h);
-            }
-            *reinterpret_cast<ah4_t*>(kh + key * KS + 4 * c4) = h4;
-            *reinterpret_cast<ah4_t*>(kl + key * KS + 4 * c4) = l4;
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                const _Float16 h = split_hi(vr[u][x]);
-                vh[(4 * c4 + x) * VS + key] = h;
-                vl[(4 * c4 + x) * VS + key] = split_lo(vr[u][x], h);
-            }
-        }
-        __syncthreads();
-        load_tile(t0 + 16 < ce ? t0 + 16 : t0);
-
+        lds_sync();   // K is staged, V is free
         // scores: hi.hi, hi.lo and lo.hi in three accumulators
         f4_t acc[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) acc[k] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
         const _Float16* kph = kh + j * KS + 8 * g;
         const _Float16* kpl = kl + j * KS + 8 * g;
+        ah8_t Ah[3], Al[3];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            Ah[s] = *reinterpret_cast<const ah8_t*>(kph + 32 * s);
+            Al[s] = *reinterpret_cast<const ah8_t*>(kpl + 32 * s);
+        }
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            const ah8_t Ah = *reinterpret_cast<const ah8_t*>(kph + 32 * s);
-            const ah8_t Al = *reinterpret_cast<const ah8_t*>(kpl + 32 * s);
-            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, qh[s], acc[0], 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, ql[s], acc[1], 0, 0, 0);
-            acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, qh[s], acc[2], 0, 0, 0);
+            if (s + 2 < NS) {
+                Ah[(s + 2) % 3] = *reinterpret_cast<const ah8_t*>(kph + 32 * (s + 2));
+                Al[(s + 2) % 3] = *reinterpret_cast<const ah8_t*>(kpl + 32 * (s + 2));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[s % 3], qh[s], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[s % 3], ql[s], acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[s % 3], qh[s], acc[2], 0, 0, 0);
+            if (s >= 4) stage_v((s - 4) >> 1, s & 1);   // this tile's V rows
+            __builtin_amdgcn_sched_barrier(0);
         }
+        load_v(t0 + 16);
         const f4_t sc = acc[0] + (acc[1] + acc[2]);
 
         // online softmax over the tile's keys 4g + r of row j (as in attn_rows_mfma_kernel)
@@ -1516,12 +1553,11 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int kt = t0 + 4 * g + r;
-            val[r] = kt < ce && kt >= qlo && kt <= qp;
+            val[r] = (kt < ce) & (kt >= qlo) & (kt <= qp);
             sv[r] = val[r] ? a.scale * sc[r] : -INFINITY;
             mt = fmaxf(mt, sv[r]);
         }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        mt = groups_max(mt);
         const bool up = mt > m + kRowsLazy;
         const float mn = up ? mt : m;
         const float alpha = !up ? 1.0f : m == -INFINITY ? 0.0f : expf(m - mn);
@@ -1537,8 +1573,6 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
 #pragma unroll
             for (int b = 0; b < NB; b++) o[b] *= alpha;
         }
-
-        // O^T += V^T . P^T
         ah4_t Ph, Pl;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -1547,14 +1581,39 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
             Ph[r] = h;
             Pl[r] = split_lo(p16, h);
         }
+        lds_sync();   // V is staged, K is free
+
+        // O^T += V^T . P^T, four blocks at a time so that no product waits for the
+        // one before it
+        const _Float16* vph = vh + j * 16 + 4 * (g ^ (2 * (j >> 3)));
+        const _Float16* vpl = vl + j * 16 + 4 * (g ^ (2 * (j >> 3)));
+        ah4_t Vh[2][4], Vl[2][4];
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            const ah4_t Vh = *reinterpret_cast<const ah4_t*>(vh + (16 * b + j) * VS + 4 * g);
-            const ah4_t Vl = *reinterpret_cast<const ah4_t*>(vl + (16 * b + j) * VS + 4 * g);
-            o[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(Vh, Ph, o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(Vh, Pl, o[b], 0, 0, 0);
-            o[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(Vl, Ph, o[b], 0, 0, 0);
+        for (int u = 0; u < 4; u++) {
+            Vh[0][u] = *reinterpret_cast<const ah4_t*>(vph + 256 * u);
+            Vl[0][u] = *reinterpret_cast<const ah4_t*>(vpl + 256 * u);
         }
+#pragma unroll
+        for (int b = 0; b < NB; b += 4) {
+            const int cu = (b >> 2) & 1;
+            if (b + 4 < NB) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    Vh[cu ^ 1][u] = *reinterpret_cast<const ah4_t*>(vph + 256 * (b + 4 + u));
+                    Vl[cu ^ 1][u] = *reinterpret_cast<const ah4_t*>(vpl + 256 * (b + 4 + u));
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; u++) o[b + u] = __builtin_amdgcn_mfma_f32_16x16x16f16(Vh[cu][u], Ph, o[b + u], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; u++) o[b + u] = __builtin_amdgcn_mfma_f32_16x16x16f16(Vh[cu][u], Pl, o[b + u], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; u++) o[b + u] = __builtin_amdgcn_mfma_f32_16x16x16f16(Vl[cu][u], Ph, o[b + u], 0, 0, 0);
+            stage_k(b >> 2);   // the next tile's K rows
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        load_k(t0 + 32);
     }
 
     lsum += __shfl_xor(lsum, 16);
@@ -1604,8 +1663,6 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(H
 // issue (half of the time) and the matrix cores (a quarter), which a wave
 // overlaps only in part.
 constexpr int kR5Keys = 32, kR5KRow = 2080;
-typedef __attribute__((address_space(1))) const f2_t g4_gf2_t;
-typedef h2v_t ah2_t;
 
 // e^x for x <= kRowsLazy, 0 below the smallest normal number: 2^(x log2 e) with
 // the product's rounding error put back to first order (within 2 ulp)
@@ -1615,7 +1672,6 @@ __device__ __forceinline__ float exp_le(float x) {
     const float e = __builtin_amdgcn_exp2f(t);
     return __builtin_fmaf(e, r * 0.693147181f, e);
 }
-__device__ __forceinline__ ah4_t join4(ah2_t a, ah2_t b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3); }
 
 // exponent field f of the scale 2^(f - 127) that brings mx into [2^14, 2^15)
 // (clamped so that 16 times its inverse 2^(127 - f) inverts again)
@@ -1809,10 +1865,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
                 mt = fmaxf(mt, sv[e]);
             }
         }
-        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-        et = fmaxf(et, __shfl_xor(et, 16, 64));
-        et = fmaxf(et, __shfl_xor(et, 32, 64));   // the tile's largest factor, the same in every lane
+        mt = groups_max(mt);
+        et = groups_max(et);   // the tile's largest factor, the same in every lane
         const bool up = mt > m + kRowsLazy;   // as in attn_rows_mfma_kernel
         const float mn = up ? mt : m;
         const float En = fmaxf(E, et);
