@@ -297,6 +297,8 @@ __global__ __launch_bounds__(64 * RW) void mm_batch_f32_kernel(const uint16_t* _
 }
 
 // ---- Q6_K weights -----------------------------------------------------------
+// A row group's next weights are loaded once its last group has been decoded, into
+// the same registers; the other wave of the SIMD covers the wait.
 // The activations come by global -> LDS copies of whole 128-byte lines, eight
 // lines an instruction: an instruction costs the L1 four cycles for every line
 // it touches, and loads straight into operand order (a 16-byte piece of 32 lines)
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(64 * RW) void mm_batch_f32_kernel(const uint16_t* _
 __device__ __forceinline__ int line_swz(int t) { return ((t >> 1) & 1) | ((t >> 2) & 2); }
 
 template <int NT, int RT, int NS>
-__global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1 : 2))) void mm_batch_q6_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                           float* __restrict__ out, int n, int d, int m, int vec) {
     static_assert(NS == 2 || NS == 4, "a block's four groups use the stages in turn");
     constexpr int kGroup = 4096 * NT;     // bytes of a group of the tile's tokens
@@ -361,15 +363,13 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
         uint2 sc[RT];
         uint32_t dh[RT];
     };
-    auto load_w = [&](int b, WRaw& r) {
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
-            r.ql[rt][0] = buf_load16(rql, (int)(rB[rt] * 128 + 32 * g), b * 128);
-            r.ql[rt][1] = buf_load16(rql, (int)(rB[rt] * 128 + 32 * g + 16), b * 128);
-            r.qh[rt] = buf_load16(rqh, (int)(rB[rt] * 64 + 16 * g), b * 64);
-            r.sc[rt] = buf_load8(rsc, (int)(rB[rt] * 16 + 8 * h), b * 16);
-            r.dh[rt] = __builtin_amdgcn_raw_buffer_load_b16(rd, (int)(rB[rt] * 2), b * 2, 0);
-        }
+    WRaw wr;
+    auto load_w = [&](int b, int rt) {
+        wr.ql[rt][0] = buf_load16(rql, (int)(rB[rt] * 128 + 32 * g), b * 128);
+        wr.ql[rt][1] = buf_load16(rql, (int)(rB[rt] * 128 + 32 * g + 16), b * 128);
+        wr.qh[rt] = buf_load16(rqh, (int)(rB[rt] * 64 + 16 * g), b * 64);
+        wr.sc[rt] = buf_load8(rsc, (int)(rB[rt] * 16 + 8 * h), b * 16);
+        wr.dh[rt] = __builtin_amdgcn_raw_buffer_load_b16(rd, (int)(rB[rt] * 2), b * 2, 0);
     };
 
     f4_t acc[RT][NT];
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
         for (int nt = 0; nt < NT; nt++) acc[rt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
     const h2_t m1056 = {(_Float16)-1056.0f, (_Float16)-1056.0f};
 
-    auto group = [&](int st, int k, const WRaw& wc, const float (&dw)[RT][4]) {
+    auto group = [&](int st, int k, int bn, const float (&dw)[RT][4]) {
         h8_t Xh[2][NT], Xl[2][NT];
         float ts[NT];
 #pragma unroll
@@ -414,16 +414,16 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             const int sb = 2 * k + s;   // sub-block 8 h + 2 k + s
-            const _Float16 scf = (_Float16)(float)(int)(int8_t)byte_of(sb < 4 ? wc.sc[rt].x : wc.sc[rt].y, sb & 3);
+            const _Float16 scf = (_Float16)(float)(int)(int8_t)byte_of(sb < 4 ? wr.sc[rt].x : wr.sc[rt].y, sb & 3);
             const h2_t SC = {scf, scf};
             f4_t S[NT];
 #pragma unroll
             for (int half = 0; half < 2; half++) {
                 // codes of step 2 k + half: ql bytes 16 half + 8 (k & 1) + t, nibble
                 // k >> 1; qh bytes 8 half + t, bits 2 k .. 2 k + 1
-                const uint4 L = wc.ql[rt][half];
+                const uint4 L = wr.ql[rt][half];
                 const uint32_t l0 = (k & 1) ? L.z : L.x, l1 = (k & 1) ? L.w : L.y;
-                const uint32_t h0 = half ? wc.qh[rt].z : wc.qh[rt].x, h1 = half ? wc.qh[rt].w : wc.qh[rt].y;
+                const uint32_t h0 = half ? wr.qh[rt].z : wr.qh[rt].x, h1 = half ? wr.qh[rt].w : wr.qh[rt].y;
                 const uint32_t q0 = ((l0 >> (4 * (k >> 1))) & 0x0f0f0f0fu) | (((h0 >> (2 * k)) & 0x03030303u) << 4);
                 const uint32_t q1 = ((l1 >> (4 * (k >> 1))) & 0x0f0f0f0fu) | (((h1 >> (2 * k)) & 0x03030303u) << 4);
                 const h2_t v0 = bits_h2(__builtin_amdgcn_perm(kMagic, q0, kSelLo)) + m1056;
@@ -443,6 +443,7 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++) S[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Wb, Xh[half][nt], S[nt], 0, 0, 0);
             }
+            if (k == 3) load_w(bn, rt);   // the row group's next block, into the registers just read
 #pragma unroll
             for (int nt = 0; nt < NT; nt++)
 #pragma unroll
@@ -450,12 +451,12 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
                     acc[rt][nt][v] = __builtin_fmaf(S[nt][v] * ts[nt], dw[rt][v], acc[rt][nt][v]);
         }
     };
-    auto block = [&](int b, const WRaw& wc, WRaw& wn) {
+    auto block = [&](int b) {
         const int bn = b + 4 < nb ? b + 4 : b;   // (the last block again at the end: no branch around the loads)
         float dw[RT][4];                         // d of rows 4 g + v
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
-            const float dl = hbits_to_f32(wc.dh[rt]);
+            const float dl = hbits_to_f32(wr.dh[rt]);
 #pragma unroll
             for (int v = 0; v < 4; v++) dw[rt][v] = __shfl(dl, 4 * g + v, 64);
         }
@@ -470,19 +471,15 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
             __builtin_amdgcn_sched_barrier(0);   // (a group's operands are not formed ahead of it)
             constexpr int kAhead = NS - 1;
             copy_x(k + kAhead < 4 ? b : bn, (k + kAhead) & 3, (k + kAhead) & (NS - 1));
-            if (k == 0) load_w(bn, wn);
-            group(k & (NS - 1), k, wc, dw);
+            group(k & (NS - 1), k, bn, dw);
         }
     };
     if (wave < nb) {
-        WRaw w0, w1;
-        load_w(wave, w0);
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) load_w(wave, rt);
 #pragma unroll
         for (int k = 0; k < NS - 1; k++) copy_x(wave, k, k);
-        for (int b = wave; b < nb; b += 8) {
-            block(b, w0, w1);
-            if (b + 4 < nb) block(b + 4, w1, w0);
-        }
+        for (int b = wave; b < nb; b += 4) block(b);
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the last copies, read by nobody, land before the sums go there
     __syncthreads();
@@ -502,11 +499,12 @@ __global__ __launch_bounds__(256) void mm_batch_q6_kernel(const uint8_t* __restr
 // load straight into operand order, and the fp32 matrix cores before:
 //   bf16 10752 x 2560, 512 tokens: 64 x 128 tiles 133 (155, 307), 64 x 64 167; 130
 //     tokens 45 (52, 106); 37 tokens, 64 x 64 28 (32, 55); 6 tokens, 16 x 16 17 (18, 42)
-//   Q6_K 2560 x 10240, 512 tokens: 32 x 80 tiles 164 (167, 344), 16 x 16 454; 130
-//     tokens, 32 x 64 65 (71, 139); 37 tokens, 16 x 32 32 (38, 94); 6 tokens, 16 x 16
-//     23 (23, 92)
-// The large Q6_K tile holds 460 registers: one wave a SIMD, whose splits, decode
-// and products overlap only in part (64 x 80 tiles spill: 216 us and more).
+//   Q6_K 2560 x 10240, 512 tokens: 64 x 80 tiles 138, 32 x 80 (two a CU) 153 on that
+//     box, 134 on another (167, 344); 384 tokens 64 x 64 111, 32 x 80 131; 130 tokens,
+//     32 x 64 66 (71, 139); 37 tokens, 16 x 32 31 (38, 94); 6 tokens, 16 x 16 23 (23, 92).
+//     VALU issue (splits and decode) and the products share the SIMDs; with the next
+//     block's weights loaded into a second set of registers the 32 x 80 tile held 460
+//     of them, one wave a SIMD, and took 164.
 struct Tile {
     int nt, rt, cost;
     void (*launch)(const void* w, const float* x, float* o, int n, int d, int m);
@@ -527,11 +525,9 @@ void launch_q6(const void* w, const float* x, float* o, int n, int d, int m) {
 
 const Tile kTilesBf16[] = {{1, 1, 5, launch_bf16<1, 1>},  {1, 2, 8, launch_bf16<1, 2>},  {2, 4, 16, launch_bf16<2, 4>},
                            {4, 4, 28, launch_bf16<4, 4>}, {4, 6, 35, launch_bf16<4, 6>}, {4, 8, 44, launch_bf16<4, 8>}};
-const Tile kTilesQ6[] = {{1, 1, 20, launch_q6<1, 1, 4>},
-                         {1, 2, 27, launch_q6<1, 2, 4>},
-                         {2, 2, 43, launch_q6<2, 2, 4>},
-                         {2, 4, 65, launch_q6<2, 4, 4>},
-                         {2, 5, 81, launch_q6<2, 5, 4>}};
+const Tile kTilesQ6[] = {{1, 1, 20, launch_q6<1, 1, 4>},  {1, 2, 26, launch_q6<1, 2, 4>}, {2, 2, 41, launch_q6<2, 2, 2>},
+                         {2, 4, 62, launch_q6<2, 4, 2>},  {2, 5, 75, launch_q6<2, 5, 2>}, {4, 4, 110, launch_q6<4, 4, 2>},
+                         {4, 5, 130, launch_q6<4, 5, 2>}};
 
 template <int N>
 const Tile& pick_tile(const Tile (&tiles)[N], int d, int m) {
