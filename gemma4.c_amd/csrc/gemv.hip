@@ -913,6 +913,138 @@ __global__ __launch_bounds__(PRO ? 64 * NB : 64) void gemv_q45_stream_kernel(con
     }
 }
 
+// Rows longer than one wave's blocks: the NW waves of a workgroup take BPW
+// consecutive blocks each of the same 8 / NMAT rows, all loads issued at once as
+// in gemv_q45_stream_kernel, and leave every block's integer sums and scales per
+// lane in LDS; wave 0 then runs the reference's fp32 chain over the blocks in
+// order (the same bits).  The Q8_K blocks of a wave are staged by the wave.
+// Bound by the wait for one wave's loads and the chain over the blocks: the
+// rows kernel keeps 32 lane groups on 32 rows, so few rows leave most CUs with
+// nothing in flight.  Q4_K, nb 12 / 28 / 40 at 4096 rows 7.6 / 19.8 / 27.0 ->
+// 5.2 / 9.3 / 10.6 us, 500 rows of 40 blocks 18.8 -> 6.2; gate|up of nb 12 at
+// 8192 rows 16.5 -> 9.8; 60000 rows of 11 blocks 25.3 -> 22.6 (4.2 TB/s).
+template <bool Q5, int BPW, int NMAT>
+__global__ __launch_bounds__(320) void gemv_q45_kwave_kernel(const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1,
+                                                             const uint8_t* __restrict__ q8, float* __restrict__ out, int nb,
+                                                             int d, const float* __restrict__ aux) {
+    constexpr int RPW = 8 / NMAT;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane & 7, k = l & 3;
+    const int nw = blockDim.x >> 6;
+    const int grp = (lane >> 3) & (RPW - 1), m = NMAT == 2 ? lane >> 5 : 0;
+    const int r0 = blockIdx.x * RPW, row = min(r0 + grp, d - 1);
+    const uint32_t nblk = (uint32_t)d * nb;
+    const uint32_t hdr_off = (Q5 ? 160u : 128u) * nblk, qh_off = 128u * nblk;
+    float4* terms = reinterpret_cast<float4*>(smem);                        // [nw BPW][64]
+    uint8_t* sq = smem + (size_t)nw * BPW * 1024 + wv * (BPW * 288 + 64);   // this wave's codes and bsums
+    const int b0 = wv * BPW;
+    // the wave's Q8_K: codes 16 BPW pieces, bsums 2 BPW (blocks past the row
+    // repeat its last one, unused)
+    constexpr int QPL = (16 * BPW + 63) / 64;
+    uint4 qv[QPL], bv = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int j = 0; j < QPL; j++) {
+        const int c = min(lane + 64 * j, 16 * BPW - 1);
+        qv[j] = reinterpret_cast<const uint4*>(q8)[min(b0 + (c >> 4), nb - 1) * 16 + (c & 15)];
+    }
+    {
+        const int c = min(lane, 2 * BPW - 1);
+        bv = reinterpret_cast<const uint4*>(q8 + q8k_bsums_off(nb))[min(b0 + (c >> 1), nb - 1) * 2 + (c & 1)];
+    }
+    const uint8_t* const wm = m ? w1 : w0;
+    const uint32_t rb = (uint32_t)row * nb;
+    uint4 wq[BPW], hd[BPW];
+    uint32_t qh[BPW];
+    float yd[BPW];
+#pragma unroll
+    for (int u = 0; u < BPW; u++) yd[u] = reinterpret_cast<const float*>(q8 + q8k_d_off(nb))[min(b0 + u, nb - 1)];
+#pragma unroll
+    for (int u = 0; u < BPW; u++) {
+        const uint32_t b = (uint32_t)min(b0 + u, nb - 1);
+        wq[u] = *reinterpret_cast<const uint4*>(wm + (rb + b) * 128u + 16 * l);
+        hd[u] = *reinterpret_cast<const uint4*>(wm + hdr_off + (rb + b) * 16u);
+        qh[u] = Q5 ? *reinterpret_cast<const uint32_t*>(wm + qh_off + (rb + b) * 32u + 4 * l) : 0u;
+    }
+    __builtin_amdgcn_sched_barrier(0);   // all loads issued before the LDS stores wait for the first ones
+#pragma unroll
+    for (int j = 0; j < QPL; j++) {
+        const int c = lane + 64 * j;
+        if (c < 16 * BPW) reinterpret_cast<uint4*>(sq)[c] = qv[j];
+    }
+    if (lane < 2 * BPW) reinterpret_cast<uint4*>(sq + BPW * 256)[lane] = bv;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the wave's own)
+    const uint32_t selA = (k & 1) ? 0x0c020c02u : 0x0c000c00u;
+    const uint32_t selB = (k & 1) ? 0x0c030c03u : 0x0c010c01u;
+    const uint32_t kmask = k < 2 ? 0xffffffffu : 0u;
+#pragma unroll
+    for (int u = 0; u < BPW; u++) {
+        const uint4 a0 = *reinterpret_cast<const uint4*>(sq + 32 * l + u * 256);
+        const uint4 a1 = *reinterpret_cast<const uint4*>(sq + 32 * l + u * 256 + 16);
+        const uint2 bsw = *reinterpret_cast<const uint2*>(sq + BPW * 256 + u * 32 + 8 * k);
+        const uint32_t sc_lo = hd[u].y & 0x3f3f3f3fu;
+        const uint32_t sc_hi = (hd[u].w & 0x0f0f0f0fu) | (((hd[u].y >> 6) & 0x03030303u) << 4);
+        const uint32_t mn_lo = hd[u].z & 0x3f3f3f3fu;
+        const uint32_t mn_hi = ((hd[u].w >> 4) & 0x0f0f0f0fu) | (((hd[u].z >> 6) & 0x03030303u) << 4);
+        const uint32_t mnw = (mn_lo & kmask) | (mn_hi & ~kmask);
+        int32_t sumi = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t qw = word_of(wq[u], j);
+            uint32_t lo = qw & 0x0f0f0f0fu, hi = (qw >> 4) & 0x0f0f0f0fu;
+            if (Q5) {
+                lo |= ((qh[u] >> (2 * j)) & 0x01010101u) << 4;
+                hi |= ((qh[u] >> (2 * j + 1)) & 0x01010101u) << 4;
+            }
+            const int dl = __builtin_amdgcn_sdot4((int)lo, (int)word_of(a0, j), 0, false);
+            const int dh = __builtin_amdgcn_sdot4((int)hi, (int)word_of(a1, j), 0, false);
+            const uint32_t pk = __builtin_amdgcn_perm((uint32_t)dh, (uint32_t)dl, 0x05040100u);
+            const uint32_t scp = __builtin_amdgcn_perm(0u, j < 2 ? sc_lo : sc_hi, (j & 1) ? 0x0c030c02u : 0x0c010c00u);
+            sumi = dot2_i16(pk, scp, sumi);
+        }
+        int32_t P = dot2_i16(bsw.x, __builtin_amdgcn_perm(0u, mnw, selA),
+                             dot2_i16(bsw.y, __builtin_amdgcn_perm(0u, mnw, selB), 0));
+        if (Q5) {
+            int32_t pm = l < 4 ? P : 0;
+            pm += __shfl_xor(pm, 1, 64);
+            pm += __shfl_xor(pm, 2, 64);
+            P = __shfl(pm, lane & ~7, 64);
+        }
+        terms[(b0 + u) * 64 + lane] = make_float4(yd[u] * half_bits_to_f32(hd[u].x & 0xffffu), (float)sumi,
+                                                  -yd[u] * half_bits_to_f32(hd[u].x >> 16), (float)P);
+    }
+    __syncthreads();
+    if (wv) return;
+    float acc = 0.0f, accm = 0.0f, summs = 0.0f;
+#pragma unroll 8
+    for (int b = 0; b < nb; b++) {
+        const float4 t = terms[b * 64 + lane];
+        acc = __builtin_fmaf(t.x, t.y, acc);
+        if (Q5) {
+            const float tm = t.z * t.w;
+            summs = summs + tm;
+        } else if (l < 4) {
+            accm = __builtin_fmaf(t.z, t.w, accm);
+        }
+    }
+    const float t1 = acc + __shfl_xor(acc, 4, 64);
+    const float t2 = t1 + __shfl_xor(t1, 2, 64);
+    const float h = t2 + __shfl_xor(t2, 1, 64);
+    float r;
+    if (Q5) {
+        r = h + summs;
+    } else {
+        const float v1 = accm + __shfl_xor(accm, 2, 64);
+        r = h + (v1 + __shfl_xor(v1, 1, 64));
+    }
+    const int ro = r0 + grp;
+    if (NMAT == 2) {
+        const float up = __shfl_xor(r, 32, 64);
+        if (l == 0 && m == 0 && ro < d) out[ro] = gelu_ref(r) * up;
+    } else if (l == 0 && ro < d) {
+        out[ro] = aux ? gelu_ref(r) * aux[ro] : r;
+    }
+}
+
 // ------------------------------------------------------------------------
 // Q6_K x fp32 (mm_quant_rows semantics), one row slice per 8-lane group
 // ------------------------------------------------------------------------
@@ -1112,7 +1244,7 @@ using namespace g4;
 // ------------------------------------------------------------------------
 // Q6_K x fp32, one K slice per 8-lane group (rows of up to 64 blocks)
 // ------------------------------------------------------------------------
-// Group g of a workgroup of 8*nb threads owns block g of every row, so the
+// Group g of a workgroup of 8*nb threads (whole waves) owns block g of every row, so the
 // 32 elements of x its lanes use (lane L = 4h+u: 128h + 32k + 8u + e, the
 // mapping of gemv_q6k_rows_kernel) and their run sums stay in registers:
 // no staging of x through LDS and no LDS reads in the loop.  A workgroup
@@ -1126,6 +1258,7 @@ namespace g4 {
 
 constexpr int kQ6SliceRows = 5;       // 512 workgroups at the FFN-down shape: two per CU
 constexpr int kQ6SliceMaxNb = 64;
+constexpr int kQ6SliceIdleRows = 40000;
 
 template <int R>
 __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(const uint8_t* __restrict__ w,
@@ -1135,6 +1268,7 @@ __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(cons
     const int tid = threadIdx.x, L = tid & 7, g = tid >> 3, h = L >> 2, u = L & 3;
     const int r0 = blockIdx.x * R;
     const Q6KPlanes P = q6k_planes((size_t)d * nb);
+    const int gb = min(g, nb - 1);   // (whole waves: groups past the row repeat its last block, unused)
     // x of this lane first (runs k = 0..3 of 8 elements at g*256 + 128h +
     // 32k + 8u), then every weight load of the R rows, all issued before
     // anything waits: the load counter retires in order, so the run sums
@@ -1142,7 +1276,7 @@ __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(cons
     float4 xa[4], xb[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const float4* xp = reinterpret_cast<const float4*>(x + (size_t)g * 256 + 128 * h + 32 * k + 8 * u);
+        const float4* xp = reinterpret_cast<const float4*>(x + (size_t)gb * 256 + 128 * h + 32 * k + 8 * u);
         xa[k] = xp[0];
         xb[k] = xp[1];
     }
@@ -1151,7 +1285,7 @@ __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(cons
     uint32_t dv[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const size_t blk = (size_t)min(r0 + r, d - 1) * nb + g;
+        const size_t blk = (size_t)min(r0 + r, d - 1) * nb + gb;
         ql[r] = *reinterpret_cast<const uint4*>(w + P.ql + blk * 128 + 16 * L);
         qh[r] = *reinterpret_cast<const uint2*>(w + P.qh + blk * 64 + 8 * L);
         sc[r] = *reinterpret_cast<const uint2*>(w + P.sc + blk * 16 + 8 * h);
@@ -1468,29 +1602,59 @@ void launch_q45_pro_nm(const void* w, const void* w2, float* o, int d, const flo
     }
 }
 
-// rows of nb blocks; the split of a row over lane groups grows with the work
-// per lane (the fused gate|up pair does twice the integer work per block)
+template <bool Q5, int NB, int NMAT>
+void launch_q45_stream(const uint8_t* a, const uint8_t* b, const uint8_t* q8, float* o, int d, const float* aux) {
+    hipLaunchKernelGGL((gemv_q45_stream_kernel<Q5, NB, NMAT>), dim3((d + 8 / NMAT - 1) / (8 / NMAT)), dim3(64), 0, g4_stream(),
+                       a, b, q8, o, d, aux, ResidualArgs{});
+}
+template <bool Q5, int BPW, int NMAT>
+void launch_q45_kwave(const uint8_t* a, const uint8_t* b, const uint8_t* q8, float* o, int nb, int d, const float* aux, int nw) {
+    const size_t lds = (size_t)nw * (BPW * 1024 + BPW * 288 + 64);
+    hipLaunchKernelGGL((gemv_q45_kwave_kernel<Q5, BPW, NMAT>), dim3((d + 8 / NMAT - 1) / (8 / NMAT)), dim3(64 * nw), lds,
+                       g4_stream(), a, b, q8, o, nb, d, aux);
+}
+
+// rows of nb blocks (at most 48: check_gemv)
 template <bool Q5, int NMAT, bool DBG>
 int launch_q45(const void* w0, const void* w1, const void* q8, float* o, int nb, int d, int32_t* S, int32_t* M,
                const float* aux = nullptr) {
-    constexpr int SP = NMAT == 2 ? 4 : 2;
-    if (!DBG && (nb == 8 || nb == 10 || nb == 16)) {
-        const dim3 grid((d + 8 / NMAT - 1) / (8 / NMAT));
+    // Rows of up to 10 blocks fit one wave's registers (16 as well: 3.7 TB/s
+    // against 2.9 for the same row over two waves); longer ones go over waves of
+    // 6..10 blocks.  The rows kernel was slower at every length from 2 to 48
+    // blocks (gate|up of 8192 rows Q4_K: 4.2 / 7.9 / 12.9 -> 3.5 / 4.6 / 6.7 us
+    // at 2 / 5 / 9 blocks) and keeps single blocks, the integer sums and
+    // tensors beyond the 32-bit offsets of the streaming kernels.
+    if (!DBG && nb >= 2 && (unsigned long long)d * nb * 176 < (1ull << 32)) {
         const uint8_t* a = (const uint8_t*)w0;
         const uint8_t* b = (const uint8_t*)w1;
-        const ResidualArgs none{};
-        if (nb == 8) hipLaunchKernelGGL((gemv_q45_stream_kernel<Q5, 8, NMAT>), grid, dim3(64), 0, g4_stream(), a, b, (const uint8_t*)q8, o, d, aux, none);
-        else if (nb == 10) hipLaunchKernelGGL((gemv_q45_stream_kernel<Q5, 10, NMAT>), grid, dim3(64), 0, g4_stream(), a, b, (const uint8_t*)q8, o, d, aux, none);
-        else hipLaunchKernelGGL((gemv_q45_stream_kernel<Q5, 16, NMAT>), grid, dim3(64), 0, g4_stream(), a, b, (const uint8_t*)q8, o, d, aux, none);
-        return g4_check_launch("gemv_q45_stream_kernel");
+        const uint8_t* q = (const uint8_t*)q8;
+        if (nb <= 10 || nb == 16) {
+            switch (nb) {
+            case 2: launch_q45_stream<Q5, 2, NMAT>(a, b, q, o, d, aux); break;
+            case 3: launch_q45_stream<Q5, 3, NMAT>(a, b, q, o, d, aux); break;
+            case 4: launch_q45_stream<Q5, 4, NMAT>(a, b, q, o, d, aux); break;
+            case 5: launch_q45_stream<Q5, 5, NMAT>(a, b, q, o, d, aux); break;
+            case 6: launch_q45_stream<Q5, 6, NMAT>(a, b, q, o, d, aux); break;
+            case 7: launch_q45_stream<Q5, 7, NMAT>(a, b, q, o, d, aux); break;
+            case 8: launch_q45_stream<Q5, 8, NMAT>(a, b, q, o, d, aux); break;
+            case 9: launch_q45_stream<Q5, 9, NMAT>(a, b, q, o, d, aux); break;
+            case 10: launch_q45_stream<Q5, 10, NMAT>(a, b, q, o, d, aux); break;
+            default: launch_q45_stream<Q5, 16, NMAT>(a, b, q, o, d, aux); break;
+            }
+            return g4_check_launch("gemv_q45_stream_kernel");
+        }
+        const int nw = (nb + 9) / 10;
+        switch ((nb + nw - 1) / nw) {
+        case 6: launch_q45_kwave<Q5, 6, NMAT>(a, b, q, o, nb, d, aux, nw); break;
+        case 7: launch_q45_kwave<Q5, 7, NMAT>(a, b, q, o, nb, d, aux, nw); break;
+        case 8: launch_q45_kwave<Q5, 8, NMAT>(a, b, q, o, nb, d, aux, nw); break;
+        case 9: launch_q45_kwave<Q5, 9, NMAT>(a, b, q, o, nb, d, aux, nw); break;
+        default: launch_q45_kwave<Q5, 10, NMAT>(a, b, q, o, nb, d, aux, nw); break;
+        }
+        return g4_check_launch("gemv_q45_kwave_kernel");
     }
-    switch (nb) {   // unrolled for the row lengths of the model (256, 2048, 2560, 4096)
-    case 1: launch_q45_nb<Q5, NMAT, DBG, 1, 1>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux); break;
-    case 8: launch_q45_nb<Q5, NMAT, DBG, 8, SP>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux); break;
-    case 10: launch_q45_nb<Q5, NMAT, DBG, 10, SP>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux); break;
-    case 16: launch_q45_nb<Q5, NMAT, DBG, 16, SP>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux); break;
-    default: launch_q45_nb<Q5, NMAT, DBG, 0, 1>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux); break;
-    }
+    if (nb == 1) launch_q45_nb<Q5, NMAT, DBG, 1, 1>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux);
+    else launch_q45_nb<Q5, NMAT, DBG, 0, 1>(w0, w1, q8, o, nb, d, S, M, nullptr, nullptr, aux);
     return g4_check_launch("gemv_q45_rows_kernel");
 }
 
@@ -1523,9 +1687,17 @@ int launch_q6_xreg(const void* w, const float* x, float* o, int nb, int d, float
 template <bool SOFTCAP>
 int launch_q6_f32(const void* w, const float* x, float* o, int nb, int d, float cap) {
     if (launch_q6_xreg<SOFTCAP, false>(w, x, o, nb, d, cap, nullptr)) return g4_check_launch("gemv_q6k_xreg_kernel");
-    if (!SOFTCAP && nb <= kQ6SliceMaxNb && nb % 8 == 0) {
+    // Whole waves of lane groups.  Where over a third of them has no block of the
+    // row (nb = 1..5, 9, 10) many rows go to the rows kernel, which walks them
+    // with a grid of four workgroups per CU: 80001 rows of 3 / 9 / 10 blocks
+    // 18.3 / 34.0 / 37.7 us there, 20.2 / 37.6 / 39.4 here; 20000 rows 10.1 /
+    // 15.6 / 16.6 there, 7.3 / 12.9 / 13.2 here; 40000 rows of 10 blocks alike.
+    // The other lengths gain at every row count measured (2560 rows of 12 / 37
+    // blocks 8.5 / 13.7 -> 4.8 / 7.6 us, 40000 of 15 33.9 -> 24.7).
+    const int groups = (nb + 7) & ~7;
+    if (!SOFTCAP && nb <= kQ6SliceMaxNb && (d <= kQ6SliceIdleRows || 3 * (groups - nb) < groups)) {
         hipLaunchKernelGGL((gemv_q6k_kslice_kernel<kQ6SliceRows>), dim3((d + kQ6SliceRows - 1) / kQ6SliceRows),
-                           dim3(8 * nb), 0, g4_stream(), (const uint8_t*)w, x, o, nb, d);
+                           dim3(8 * groups), 0, g4_stream(), (const uint8_t*)w, x, o, nb, d);
         return g4_check_launch("gemv_q6k_kslice_kernel");
     }
     const int target = 2 * g4_num_cus();

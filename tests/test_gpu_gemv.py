@@ -345,6 +345,55 @@ def test_mm_quantizes_inside(lib, orc, qtype, n, d):
         assert np.array_equal(xd.to_array(np.uint32)[:d], want)
 
 
+@pytest.mark.parametrize("qtype", [12, 13])
+@pytest.mark.parametrize("nb", [2, 3, 4, 5, 6, 7, 9, 11, 12, 15, 17, 20, 21, 30, 31, 40, 41, 48])
+def test_q45_gemv_row_lengths(lib, orc, qtype, nb):
+    """Every row length in blocks (one wave, and 2 to 5 waves of 6 to 10 blocks):
+    GEMV and its gelu(.) * mul form bit for bit on mm_quant_dot_rows, gate|up on
+    the gelu of two of them (the device's tanhf against itself: same bits)."""
+    from g4 import DBuf, upload_quant
+    n = 256 * nb
+    rng = np.random.default_rng(100 * qtype + nb)
+    for d in (1, 7, 9, 37):
+        raws = [synth.rand_kquant(rng, qtype, d, n) for _ in range(2)]
+        x = (rng.standard_normal(n) * np.exp(rng.uniform(-4, 4, n))).astype(np.float32)
+        x[-256:-128] = 0.0
+        ws = [upload_quant(lib, r, qtype, n, d) for r in raws]
+        _, q8 = gpu_q8(lib, x)
+        q8h = orc.quantize_q8K(x)
+        up = DBuf(lib, 4 * d)
+        lib.g4_mm_quant_dot_rows(up.ptr, ws[1].ptr, n, d, qtype, q8.ptr)
+        want = orc.mm_quant_dot_rows(raws[1], n, d, qtype, q8h)
+        assert np.array_equal(up.to_array(np.uint32), want.view(np.uint32)), (d,)
+        a, b = DBuf(lib, 4 * d), DBuf(lib, 4 * d)
+        lib.g4_mm_quant_dot_rows_gelu_mul(a.ptr, ws[0].ptr, n, d, qtype, q8.ptr, up.ptr)
+        lib.g4_mm_gate_up_gelu(b.ptr, ws[0].ptr, ws[1].ptr, n, d, qtype, q8.ptr)
+        assert np.array_equal(a.to_array(np.uint32), b.to_array(np.uint32)), (d,)
+        g = orc.mm_quant_dot_rows(raws[0], n, d, qtype, q8h)
+        ref = np.array([orc.L.or_gelu(float(v)) for v in g], np.float32) * want
+        assert np.allclose(b.to_array(np.float32), ref, rtol=1e-5, atol=1e-6 * np.abs(ref).max()), (d,)
+
+
+@pytest.mark.parametrize("nb", [1, 2, 7, 9, 10, 11, 15, 17, 33, 47, 48])
+def test_q6K_f32_gemv_row_lengths(lib, nb):
+    """Q6_K rows whose blocks do not fill the waves, around the rows of a
+    workgroup: within the fp32 bound of a sum of n products in any order,
+    (n/8 + 16) 2^-24 sum |w x| for at most n/8 + 16 roundings on one path
+    (weights (q - 32) s formed as sum x q - 32 sum x add 127 / 31 of them)."""
+    from g4 import DBuf, upload_quant
+    n = 256 * nb
+    rng = np.random.default_rng(600 + nb)
+    for d in (1, 4, 5, 6, 41):
+        raw = synth.rand_q6K(rng, d, n)
+        x = rng.standard_normal(n).astype(np.float32)
+        w, xd, out = upload_quant(lib, raw, 14, n, d), dbuf(lib, x), DBuf(lib, 4 * d)
+        lib.g4_mm_quant_rows(out.ptr, xd.ptr, w.ptr, n, d, 14)
+        W = kq.dequant_f64(raw.reshape(-1, 210), 14).reshape(d, n)
+        x64 = x.astype(np.float64)
+        err = np.abs(out.to_array(np.float32) - W @ x64) / (np.abs(W) @ np.abs(x64))
+        assert err.max() <= min(1e-5, 5 * (n / 8 + 16) * 2.0 ** -24), (d, err.max())
+
+
 def rel_err(got, want):
     want = np.asarray(want, np.float64)
     return float(np.max(np.abs(np.asarray(got, np.float64) - want)) / max(np.max(np.abs(want)), 1e-30))
