@@ -37,8 +37,8 @@ typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
 constexpr int red_tiles(int t) { return t < 10 ? t : 10; }
 
 template <int NT, int RT, class Slow>
-__device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, float* __restrict__ out, int row0, int tok0,
-                                             int d, int m, bool vec, Slow slow) {
+__device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, int part, float* __restrict__ out, int row0,
+                                             int tok0, int d, int m, bool vec, Slow slow) {
     constexpr int T = NT * RT, R = red_tiles(T);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -46,7 +46,7 @@ __device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, flo
         if (t0) __syncthreads();
 #pragma unroll
         for (int t = t0; t < t0 + R; t++)
-            if (t < T) red[(wave * R + (t - t0)) * 64 + lane] = acc[t / NT][t % NT];
+            if (t < T) red[(part * R + (t - t0)) * 64 + lane] = acc[t / NT][t % NT];
         __syncthreads();
 #pragma unroll
         for (int t = t0; t < t0 + R; t++) {
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void mm_batch_bf16_kernel(const uint16_t* __re
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the last copies land before the sums take their place
     __syncthreads();
     f4_t* red = reinterpret_cast<f4_t*>(lds);
-    reduce_store<NT, RT>(acc, red, out, row0, tok0, d, m, vec, [&](int tok, int row) {
+    reduce_store<NT, RT>(acc, red, wave, out, row0, tok0, d, m, vec, [&](int tok, int row) {
         float sum = 0.0f;
         for (int k = 0; k < n; k++)
             sum = __builtin_fmaf(__uint_as_float((uint32_t)w[(size_t)row * n + k] << 16), x[(size_t)tok * n + k], sum);
@@ -310,8 +310,8 @@ __global__ __launch_bounds__(64 * RW) void mm_batch_f32_kernel(const uint16_t* _
 __device__ __forceinline__ int line_swz(int t) { return ((t >> 1) & 1) | ((t >> 2) & 2); }
 
 template <int NT, int RT, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1 : 2))) void mm_batch_q6_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x,
-                                                          float* __restrict__ out, int n, int d, int m, int vec) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mm_batch_q6_kernel(
+    const uint8_t* __restrict__ w, const float* __restrict__ x, float* __restrict__ out, int n, int d, int m, int vec) {
     static_assert(NS == 2 || NS == 4, "a block's four groups use the stages in turn");
     constexpr int kGroup = 4096 * NT;     // bytes of a group of the tile's tokens
     constexpr size_t kRed = sizeof(f4_t) * 4 * red_tiles(NT * RT) * 64, kStages = (size_t)4 * NS * kGroup;
@@ -322,6 +322,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1
     xcd_tile((m + 16 * NT - 1) / (16 * NT), bx, by);
     const int row0 = bx * 16 * RT, tok0 = by * 16 * NT;
     const int nb = n >> 8;
+    // the wave's part of K: workgroups that share a CU give their longer parts to different SIMDs
+    const int part = (wave + 2 * (blockIdx.x >> 8) + (blockIdx.x >> 9)) & 3;
     const size_t nblk = (size_t)d * nb;
     const Q6KPlanes P = q6k_planes(nblk);
 
@@ -474,17 +476,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1
             group(k & (NS - 1), k, bn, dw);
         }
     };
-    if (wave < nb) {
+    if (part < nb) {
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) load_w(wave, rt);
+        for (int rt = 0; rt < RT; rt++) load_w(part, rt);
 #pragma unroll
-        for (int k = 0; k < NS - 1; k++) copy_x(wave, k, k);
-        for (int b = wave; b < nb; b += 4) block(b);
+        for (int k = 0; k < NS - 1; k++) copy_x(part, k, k);
+        for (int b = part; b < nb; b += 4) block(b);
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));   // the last copies, read by nobody, land before the sums go there
     __syncthreads();
     f4_t* red = reinterpret_cast<f4_t*>(lds);
-    reduce_store<NT, RT>(acc, red, out, row0, tok0, d, m, vec, [&](int tok, int row) {
+    reduce_store<NT, RT>(acc, red, part, out, row0, tok0, d, m, vec, [&](int tok, int row) {
         float sum = 0.0f;
         for (int k = 0; k < n; k++)
             sum = __builtin_fmaf(dequant_elem(w, 14, nblk, (size_t)row * nb + (k >> 8), k & 255), x[(size_t)tok * n + k], sum);
@@ -492,21 +494,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1
     });
 }
 
-// Tile shapes.  A launch takes about ceil(workgroups / CUs) times its tile's cost;
-// the table's costs are the times of one round in us (MI355X; bf16 over 2560
-// columns, Q6_K over 10240) and the cheapest shape is taken, so small batches get
-// small tiles and more workgroups.  us, and in brackets the same tiles with every
-// load straight into operand order, and the fp32 matrix cores before:
-//   bf16 10752 x 2560, 512 tokens: 64 x 128 tiles 133 (155, 307), 64 x 64 167; 130
-//     tokens 45 (52, 106); 37 tokens, 64 x 64 28 (32, 55); 6 tokens, 16 x 16 17 (18, 42)
-//   Q6_K 2560 x 10240, 512 tokens: 64 x 80 tiles 138, 32 x 80 (two a CU) 153 on that
-//     box, 134 on another (167, 344); 384 tokens 64 x 64 111, 32 x 80 131; 130 tokens,
-//     32 x 64 66 (71, 139); 37 tokens, 16 x 32 31 (38, 94); 6 tokens, 16 x 16 23 (23, 92).
-//     VALU issue (splits and decode) and the products share the SIMDs; with the next
-//     block's weights loaded into a second set of registers the 32 x 80 tile held 460
-//     of them, one wave a SIMD, and took 164.
+// Tile shapes.  The table holds the times in us of one workgroup on a CU and of
+// two that share it, with every CU taken (MI355X, 10240 columns, a sweep of all
+// shapes over 2..512 tokens); a launch runs in rounds of two a CU and the
+// cheapest shape is taken, so small batches get small tiles and more
+// workgroups.  Two Q6_K tiles of 32 tokens x 80 rows take less than one of 64 x
+// 80 (122 against 130 us): the second wave of a SIMD covers the first one's
+// waits, and their shares of K differ (mm_batch_q6_kernel).  us, and in brackets
+// the same kernels with rounds of one a CU, where the long-K shapes took tiles of 64
+// tokens, and the fp32 matrix cores before:
+//   bf16 10752 x 2560, 512 tokens: 64 x 128 tiles 128 (128, 307); 2560 x 10240, 256
+//     tokens, 32 x 80 69 (82), 512 tokens, 64 x 96 107 (116); 10240 x 2560, 37 tokens,
+//     64 x 64 22 (25)
+//   Q6_K 2560 x 10240, 512 tokens: 32 x 80 tiles 122 (127 -- 137, 344); 10240 x 2560,
+//     512 tokens 131 -- 140 (180), 256 tokens 70 (91), 100 tokens 39 (45); 37 tokens, 16 x
+//     32 30 (31, 94); 2560 x 256, 512 tokens 10.8 (17).
+//     VALU issue (splits and decode) and the products share the SIMDs.
 struct Tile {
-    int nt, rt, cost;
+    int nt, rt, one, two;
     void (*launch)(const void* w, const float* x, float* o, int n, int d, int m);
 };
 
@@ -523,11 +528,12 @@ void launch_q6(const void* w, const float* x, float* o, int n, int d, int m) {
                        m, (int)(d % 4 == 0 && al16(o)));
 }
 
-const Tile kTilesBf16[] = {{1, 1, 5, launch_bf16<1, 1>},  {1, 2, 8, launch_bf16<1, 2>},  {2, 4, 16, launch_bf16<2, 4>},
-                           {4, 4, 28, launch_bf16<4, 4>}, {4, 6, 35, launch_bf16<4, 6>}, {4, 8, 44, launch_bf16<4, 8>}};
-const Tile kTilesQ6[] = {{1, 1, 20, launch_q6<1, 1, 4>},  {1, 2, 26, launch_q6<1, 2, 4>}, {2, 2, 41, launch_q6<2, 2, 2>},
-                         {2, 4, 62, launch_q6<2, 4, 2>},  {2, 5, 75, launch_q6<2, 5, 2>}, {4, 4, 110, launch_q6<4, 4, 2>},
-                         {4, 5, 130, launch_q6<4, 5, 2>}};
+const Tile kTilesBf16[] = {{1, 1, 37, 44, launch_bf16<1, 1>},  {1, 2, 42, 50, launch_bf16<1, 2>},
+                           {2, 2, 50, 66, launch_bf16<2, 2>},  {2, 4, 67, 101, launch_bf16<2, 4>},
+                           {2, 5, 74, 122, launch_bf16<2, 5>}, {4, 4, 89, 178, launch_bf16<4, 4>},
+                           {4, 6, 112, 224, launch_bf16<4, 6>}, {4, 8, 141, 282, launch_bf16<4, 8>}};
+const Tile kTilesQ6[] = {{1, 1, 20, 32, launch_q6<1, 1, 4>},  {1, 2, 28, 47, launch_q6<1, 2, 4>}, {2, 2, 42, 67, launch_q6<2, 2, 2>},
+                         {2, 4, 62, 100, launch_q6<2, 4, 2>}, {2, 5, 75, 122, launch_q6<2, 5, 2>}};
 
 template <int N>
 const Tile& pick_tile(const Tile (&tiles)[N], int d, int m) {
@@ -537,7 +543,8 @@ const Tile& pick_tile(const Tile (&tiles)[N], int d, int m) {
     for (int k = 0; k < N; k++) {
         const Tile& t = tiles[k];
         const long long wgs = (long long)((d + 16 * t.rt - 1) / (16 * t.rt)) * ((m + 16 * t.nt - 1) / (16 * t.nt));
-        const long long c = (wgs + cus - 1) / cus * t.cost;
+        const long long rest = wgs % (2 * cus);
+        const long long c = wgs / (2 * cus) * t.two + (rest > cus ? t.two : rest > 0 ? t.one : 0);
         if (at < 0 || c < best) best = c, at = k;
     }
     return tiles[at];

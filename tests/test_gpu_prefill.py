@@ -431,7 +431,7 @@ def test_mm_batch_f32_weights(lib, orc, qtype, n, d, m):
 
 
 @pytest.mark.parametrize("qtype", [14, 30])
-@pytest.mark.parametrize("n,d", [(256, 37), (768, 1000), (2560, 2560)])
+@pytest.mark.parametrize("n,d", [(256, 37), (768, 1000), (2560, 2560), (1280, 4099)])
 def test_mm_batch_f32_tiles(lib, qtype, n, d):
     """Every tile shape of the Q6_K / bf16 GEMM on fp32 activations (batches of
     1 to 600 tokens, rows that end inside a tile, an output that is only
