@@ -1352,8 +1352,8 @@ __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(cons
 // covers kXrRpi rows; eight passes make a batch of 8*kXrRpi rows whose
 // block partials (each summed over its 8 lanes) go to LDS; after a barrier
 // one thread per row in one wave (a different wave each batch) add each row's NB
-// partials, apply the soft-cap, store and (AM) keep the argmax key.  Batches are dealt to the workgroups round
-// robin (d a multiple of the batch); each thread keeps kXrPf
+// partials, apply the soft-cap, store and (AM) keep the argmax key.  Batches
+// are dealt to the workgroups round robin; each thread keeps kXrPf
 // passes of weight loads in flight (past the last pass: the last one again,
 // so no load sits under a branch).
 // Same per-block arithmetic as gemv_q6k_rows_kernel (fp32 tolerance of the
@@ -1372,7 +1372,7 @@ __global__ __launch_bounds__(8 * NB * kXrRpi) void gemv_q6k_xreg_kernel(const ui
     __shared__ __align__(16) float part[2][BR][kXrRow];
     __shared__ unsigned long long red[NT / 64];
     const int t = threadIdx.x, r = t / (8 * NB), s = t - r * (8 * NB), b = s >> 3, L = s & 7, h = L >> 2, u = L & 3;
-    const int nbatch = d / BR;
+    const int nbatch = (d + BR - 1) / BR;
     const int mine = (int)blockIdx.x < nbatch ? (nbatch - 1 - (int)blockIdx.x) / (int)gridDim.x + 1 : 0;
     const int nsteps = 8 * mine;
     unsigned long long best = 0;   // argmax key of this thread's rows
@@ -1391,13 +1391,15 @@ __global__ __launch_bounds__(8 * NB * kXrRpi) void gemv_q6k_xreg_kernel(const ui
             uint2 qh, sc;
             uint32_t dv;
         };
-        // a pass's first block (uniform) plus this thread's offsets: the rows
-        // are whole batches (d a multiple of BR), so no row is clamped
+        // a pass's first block (uniform) plus this thread's offsets
         const uint32_t rb = (uint32_t)(r * NB + b);
         const uint32_t o_ql = rb * 128u + 16u * L, o_qh = rb * 64u + 8u * L, o_sc = rb * 16u + 8u * h, o_d = rb * 2u;
+        // first row of step j's batch: the last one ends at the last row (rows it
+        // shares with the batch before are computed twice, to the same bits)
+        auto row0 = [&](int j) { return min(((int)blockIdx.x + (j >> 3) * (int)gridDim.x) * BR, d - BR); };
         auto load = [&](int j, Wt& q) {
             j = min(j, nsteps - 1);
-            const size_t pb = ((size_t)((int)blockIdx.x + (j >> 3) * (int)gridDim.x) * BR + (j & 7) * kXrRpi) * NB;
+            const size_t pb = (size_t)(row0(j) + (j & 7) * kXrRpi) * NB;
             q.ql = *reinterpret_cast<const uint4*>(w + P.ql + pb * 128 + o_ql);
             q.qh = *reinterpret_cast<const uint2*>(w + P.qh + pb * 64 + o_qh);
             q.sc = *reinterpret_cast<const uint2*>(w + P.sc + pb * 16 + o_sc);
@@ -1465,7 +1467,7 @@ __global__ __launch_bounds__(8 * NB * kXrRpi) void gemv_q6k_xreg_kernel(const ui
                         for (int m = 1; m < NB; m <<= 1)
 #pragma unroll
                             for (int i = 0; i + m < NB; i += 2 * m) v[i] += v[i + m];
-                        const int row = ((int)blockIdx.x + (j >> 3) * (int)gridDim.x) * BR + tr;
+                        const int row = row0(j) + tr;
                         const float o = SOFTCAP ? cap * tanhf(v[0] * inv) : v[0];
                         out[row] = o;
                         if (AM) {
@@ -1670,24 +1672,52 @@ void launch_q6_ks(const void* w, const float* x, float* o, int nb, int d, float 
                        (const uint8_t*)w, x, o, nb, d, cap, nullptr);
 }
 
-// the register-x kernel for rows of 10 blocks (the LM head at hidden 2560)
-// once there are enough rows for two workgroups per CU; returns the grid,
-// 0 when it does not apply
-constexpr int kXrWgPerCu = 1;
-template <bool SOFTCAP, bool AM>
-int launch_q6_xreg(const void* w, const float* x, float* o, int nb, int d, float cap, unsigned long long* part) {
-    const int nbatch = d / (8 * kXrRpi);
-    const int grid = kXrWgPerCu * g4_num_cus();
-    if (nb != 10 || d % (8 * kXrRpi) || nbatch < grid) return 0;
-    hipLaunchKernelGGL((gemv_q6k_xreg_kernel<10, SOFTCAP, AM>), dim3(grid), dim3(8 * 10 * kXrRpi), 0, g4_stream(),
+// the register-x kernel for rows of 4..12 blocks once there is a batch of rows
+// for every CU; returns the grid, 0 when it does not apply.  Workgroups per CU:
+// one of 576 threads and more, two small ones (and mid-sized ones in long launches).
+// LM head with the argmax keys, us here / on gemv_q6k_rows_kernel: 32768 rows of 4 /
+// 7 / 10 / 12 blocks 11.5 / 15.4 / 20.0 / 22.3 here, 18.1 / 20.8 / 25.8 / 30.8 there,
+// 262144 rows 44.6 / 72.6 / 105.7 / 116 here, 51.8 / 87.5 / 111.6 / 138 there.
+constexpr int kXrLongRows = 131072;
+int xreg_wg_per_cu(int nb, int d) { return nb <= 5 || (nb <= 8 && d >= kXrLongRows) ? 2 : 1; }
+int xreg_batches(int d) { return (d + 8 * kXrRpi - 1) / (8 * kXrRpi); }
+template <int NB, bool SOFTCAP, bool AM>
+int launch_q6_xreg_nb(const void* w, const float* x, float* o, int d, float cap, unsigned long long* part) {
+    const int grid = min(xreg_wg_per_cu(NB, d) * g4_num_cus(), xreg_batches(d));
+    hipLaunchKernelGGL((gemv_q6k_xreg_kernel<NB, SOFTCAP, AM>), dim3(grid), dim3(8 * NB * kXrRpi), 0, g4_stream(),
                        (const uint8_t*)w, x, o, d, cap, part);
     return grid;
+}
+template <bool SOFTCAP, bool AM>
+int launch_q6_xreg(const void* w, const float* x, float* o, int nb, int d, float cap, unsigned long long* part) {
+    if (d < 8 * kXrRpi * g4_num_cus()) return 0;
+    if (!AM && !SOFTCAP) {
+        // against gemv_q6k_kslice_kernel: only with the last round three quarters full
+        // (20001 rows of 10 blocks 15.3 here, 13.2 there), and rows of 6..8 blocks
+        // only in long launches (50001 rows 18.4-20.5 here, 16.4-18.0 there; 262144
+        // 60-75 here, 73-78 there); 32768 rows of 4 / 9 / 12 blocks 8.4 / 15.4 / 18.3
+        // here, 10.5 / 19.2 / 20.1 there
+        const int per = xreg_wg_per_cu(nb, d) * g4_num_cus(), rounds = (xreg_batches(d) + per - 1) / per;
+        if ((nb >= 6 && nb <= 8 && d < kXrLongRows) || 4 * xreg_batches(d) < 3 * rounds * per) return 0;
+    }
+    switch (nb) {
+    case 4: return launch_q6_xreg_nb<4, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 5: return launch_q6_xreg_nb<5, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 6: return launch_q6_xreg_nb<6, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 7: return launch_q6_xreg_nb<7, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 8: return launch_q6_xreg_nb<8, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 9: return launch_q6_xreg_nb<9, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 10: return launch_q6_xreg_nb<10, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 11: return launch_q6_xreg_nb<11, SOFTCAP, AM>(w, x, o, d, cap, part);
+    case 12: return launch_q6_xreg_nb<12, SOFTCAP, AM>(w, x, o, d, cap, part);
+    default: return 0;
+    }
 }
 
 template <bool SOFTCAP>
 int launch_q6_f32(const void* w, const float* x, float* o, int nb, int d, float cap) {
     if (launch_q6_xreg<SOFTCAP, false>(w, x, o, nb, d, cap, nullptr)) return g4_check_launch("gemv_q6k_xreg_kernel");
-    // Whole waves of lane groups.  Where over a third of them has no block of the
+    // What the register-x kernel leaves, in whole waves of lane groups.  Where over a third of them has no block of the
     // row (nb = 1..5, 9, 10) many rows go to the rows kernel, which walks them
     // with a grid of four workgroups per CU: 80001 rows of 3 / 9 / 10 blocks
     // 18.3 / 34.0 / 37.7 us there, 20.2 / 37.6 / 39.4 here; 20000 rows 10.1 /

@@ -394,6 +394,38 @@ def test_q6K_f32_gemv_row_lengths(lib, nb):
         assert err.max() <= min(1e-5, 5 * (n / 8 + 16) * 2.0 ** -24), (d, err.max())
 
 
+@pytest.mark.parametrize("nb,d", [(4, 16384), (5, 32769), (6, 131073), (7, 16447), (8, 20001), (9, 16385), (10, 32700),
+                                  (11, 32769), (12, 16399)])
+def test_q6K_register_x_row_lengths(lib, orc, nb, d):
+    """The register-x kernel at each row length, row counts that end inside a
+    batch of 64: outputs to the GEMV bar, with the soft-cap (derivative <= 1) and
+    without, and the argmax key the first index of the largest output."""
+    from g4 import DBuf, upload_quant
+    n, cap = 256 * nb, 30.0
+    rng = np.random.default_rng(nb + d)
+    raw = synth.rand_q6K(rng, d, n)
+    x = rng.standard_normal(n).astype(np.float32)
+    w, xd = upload_quant(lib, raw, 14, n, d), dbuf(lib, x)
+    want, mag = orc.mm_quant_rows(x, raw, n, d, 14).astype(np.float64), kq.abs_dot_rows(raw, 14, n, x)
+    out, tok = DBuf(lib, 4 * (d + 1)), DBuf(lib, 4)
+    part = DBuf(lib, lib.L.g4_mm_argmax_part_bytes(d))
+    guard = np.full(d + 1, 7.0, np.float32)
+    for c in (0.0, cap):
+        ref = cap * np.tanh(want / cap) if c else want
+        for am in (False, True):
+            out = DBuf.from_array(lib, guard)
+            if am:
+                lib.g4_mm_argmax_row(xd.ptr, w.ptr, n, d, 14, None, c, out.ptr, part.ptr, tok.ptr, None, None)
+            else:
+                lib.g4_mm_quant_rows_softcap(out.ptr, xd.ptr, w.ptr, n, d, 14, c)
+            got = out.to_array(np.float32)
+            assert got[d] == 7.0
+            err = np.abs(got[:d].astype(np.float64) - ref) - (1e-5 if c else 0.0)   # ulps of 30 cover tanhf
+            assert (err <= 1e-5 * mag).all(), (c, am)
+            if am:
+                assert int(tok.to_array(np.int32)[0]) == int(np.argmax(got[:d]))
+
+
 def rel_err(got, want):
     want = np.asarray(want, np.float64)
     return float(np.max(np.abs(np.asarray(got, np.float64) - want)) / max(np.max(np.abs(want)), 1e-30))
