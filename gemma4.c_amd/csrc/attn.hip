@@ -1641,18 +1641,23 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(2
 // for the scores (the two halves' sums meet in LDS) and for the output, so a
 // wave holds 64 registers of q and 64 of o.  32 keys a tile: both products use
 // v_mfma_f32_16x16x32_f16.
-// Range: the four K rows that a wave stages, its four V rows and every half q
-// row are scaled by the power of two that brings their largest element into
-// [2^14, 2^15) before the split (an element is then within 2^-22 of its value or
-// 2^-39 of that largest), so any finite fp32 input keeps its range.  The K
-// factor multiplies the scores; the V factor goes into its keys' weights, which
-// are kept relative to the largest factor met so far (o is scaled down when a
-// larger one comes).
+// Range: every K row, every V row and every half q row is scaled by the power of
+// two that brings its largest element into [2^14, 2^15) before the split, so an
+// element is within 2^-22 of its value or 2^-39 of its own row's largest.  The K
+// factor multiplies the key's scores; the V factor goes into the key's weights,
+// which a query row keeps relative to E, a power of two near the largest product
+// of weight and factor that it has met itself: a weight is within 2^-22 of its
+// value or 2^-29 of that product.  Neither the size of a key that a row may not see
+// nor that of one with next to no weight touches the row's other keys.  (One
+// factor for four rows and one E for the tile, masked keys among them, took 335
+// us where this takes 337 and left a row whose tile held a 2^20 times larger
+// later key 1e-3 off.)
 // LDS: K as rows of 512 hi, 512 lo (2080 bytes a row: conflict-free 16-byte
 // reads); V transposed, a 128-byte row per dim of eight 16-byte slots, slot (hl,
 // g) at (g + 4 hl) ^ (dim / 2 & 7): the keys 4g .. 4g + 3 of both 16-key halves,
 // the order in which a lane holds its weights.  Wave w stages keys 4w .. 4w + 3
-// whole, so their largest element is a reduction within the wave.
+// whole, so a row's largest element is a reduction within the wave, and the
+// four rows' reductions share their steps.
 // Two barriers a tile: V is split and staged between the score products, the
 // next tile's K between the output products, and each row's loads take the
 // registers of a row just staged (all 64 at once spilled: 470 us at the size
@@ -1678,11 +1683,29 @@ __device__ __forceinline__ float exp_le(float x) {
 __device__ __forceinline__ int scale_field(float mx) { return max(1, min(268 - (int)(__float_as_uint(mx) >> 23), 248)); }
 __device__ __forceinline__ float field_to_scale(int f) { return __uint_as_float((uint32_t)f << 23); }
 
+// the factors of four rows whose largest elements, lane by lane, are m[0..3]:
+// sf[r] for the split, uniform, and row r's inverse in every lane of group r
+__device__ __forceinline__ float rows_scale(const float (&m)[4], float (&sf)[4]) {
+    // lane group r ends up with row r; non-negative floats order as their bits
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[0]), __float_as_uint(m[2]), false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[1]), __float_as_uint(m[3]), false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(max(a[0], a[1]), max(b[0], b[1]), false, false);
+    int v = (int)max(c[0], c[1]);
+    v = max(v, dpp_i<kDppXor1>(v));
+    v = max(v, dpp_i<kDppXor2>(v));
+    v = max(v, dpp_i<kDppHalfMirror>(v));
+    v = max(v, dpp_i<kDppMirror>(v));
+    const int f = scale_field(__int_as_float(v));
+#pragma unroll
+    for (int r = 0; r < 4; r++) sf[r] = lane_f(field_to_scale(f), 16 * r);
+    return field_to_scale(254 - f);
+}
+
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void attn_rows512_kernel(AttnArgs a) {
     constexpr int HD = 512;
     __shared__ __align__(16) uint8_t ks[kR5Keys * kR5KRow];
     __shared__ __align__(16) uint8_t vs[HD * 128];
-    __shared__ __align__(16) float tsk[8], tsv[8];
+    __shared__ __align__(16) float tsk[kR5Keys], tsv[kR5Keys];
     __shared__ __align__(16) f4_t ex[8][2][64];
     const int c = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, j = lane & 15;
@@ -1727,41 +1750,43 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
         for (int k = 0; k < 4; k++) vr[r][k] = reinterpret_cast<const g4_gf2_t*>(p)[lane + 64 * k];
     };
     // staging, in parts that the products below are interleaved with
-    float ksf, vsf;
+    float ksf[4], vsf[4];
     auto scale_k = [&]() {
-        float mx = 0.0f;
+        float mx[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) {
+            mx[r] = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 2; k++) mx = max3_abs(kr[r][k][2], kr[r][k][3], max3_abs(kr[r][k][0], kr[r][k][1], mx));
-        const int f = scale_field(wave_max(mx));
-        ksf = field_to_scale(f);
-        if (lane == 0) tsk[wave] = field_to_scale(254 - f);
+            for (int k = 0; k < 2; k++) mx[r] = max3_abs(kr[r][k][2], kr[r][k][3], max3_abs(kr[r][k][0], kr[r][k][1], mx[r]));
+        }
+        const float inv = rows_scale(mx, ksf);
+        if (j == 0) tsk[4 * wave + g] = inv;
     };
     auto stage_k = [&](int r, int k) {
         uint8_t* row = ks + (4 * wave + r) * kR5KRow + 8 * lane;
         ah2_t h0, l0, h1, l1;
-        split2(kr[r][k][0], kr[r][k][1], ksf, h0, l0);
-        split2(kr[r][k][2], kr[r][k][3], ksf, h1, l1);
+        split2(kr[r][k][0], kr[r][k][1], ksf[r], h0, l0);
+        split2(kr[r][k][2], kr[r][k][3], ksf[r], h1, l1);
         *reinterpret_cast<ah4_t*>(row + 512 * k) = join4(h0, h1);
         *reinterpret_cast<ah4_t*>(row + 512 * k + 1024) = join4(l0, l1);
     };
     auto scale_v = [&]() {
-        float mx = 0.0f;
+        float mx[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) {
+            mx[r] = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 4; k++) mx = max3_abs(vr[r][k][0], vr[r][k][1], mx);
-        const int f = scale_field(wave_max(mx));
-        vsf = field_to_scale(f);
-        if (lane == 0) tsv[wave] = field_to_scale(254 - f);
+            for (int k = 0; k < 4; k++) mx[r] = max3_abs(vr[r][k][0], vr[r][k][1], mx[r]);
+        }
+        const float inv = rows_scale(mx, vsf);
+        if (j == 0) tsv[4 * wave + g] = inv;
     };
     const int kt4 = wave >> 2, kg4 = wave & 3;   // keys 16 kt4 + 4 kg4 + r
     auto stage_v = [&](int k, int x) {
         const int dim = 128 * k + 2 * lane + x, sw = lane & 7;   // sw = dim / 2 & 7
         ah2_t h0, l0, h1, l1;
-        split2(vr[0][k][x], vr[1][k][x], vsf, h0, l0);
-        split2(vr[2][k][x], vr[3][k][x], vsf, h1, l1);
+        split2(vr[0][k][x], vr[1][k][x], vsf[0], vsf[1], h0, l0);
+        split2(vr[2][k][x], vr[3][k][x], vsf[2], vsf[3], h1, l1);
         *reinterpret_cast<ah4_t*>(vs + dim * 128 + 16 * (kg4 ^ sw) + 8 * kt4) = join4(h0, h1);
         *reinterpret_cast<ah4_t*>(vs + dim * 128 + 16 * ((kg4 + 4) ^ sw) + 8 * kt4) = join4(l0, l1);
     };
@@ -1793,7 +1818,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
     }
 
     float m = -INFINITY, lsum = 0.0f;   // lsum: this lane's keys only (summed over the groups at the end)
-    float E = field_to_scale(6);        // the largest V factor met
+    float E = field_to_scale(6);        // row j's scale: o holds 16 / E of the output
     f4_t o[16];
 #pragma unroll
     for (int b = 0; b < 16; b++) o[b] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1847,12 +1872,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        const float k4[2] = {tsk[g], tsk[4 + g]};   // of keys 16 t + 4 g + r
+        // factors of keys 16 t + 4 g + r
+        const f4_t k4[2] = {*reinterpret_cast<const f4_t*>(tsk + 4 * g), *reinterpret_cast<const f4_t*>(tsk + 16 + 4 * g)};
 #pragma unroll
         for (int t = 0; t < 2; t++) ex[wave][t][lane] = (sh[t] + sx[t]) * tsq;
         lds_sync();   // both halves' sums, V is staged, K is free
-        const float v4[2] = {tsv[g], tsv[4 + g]};
-        float sv[8], mt = -INFINITY, et = fmaxf(v4[0], v4[1]);
+        const f4_t v4[2] = {*reinterpret_cast<const f4_t*>(tsv + 4 * g), *reinterpret_cast<const f4_t*>(tsv + 16 + 4 * g)};
+        float sv[8], mt = -INFINITY;
         bool val[8];
 #pragma unroll
         for (int t = 0; t < 2; t++) {
@@ -1866,32 +1892,38 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
             }
         }
         mt = groups_max(mt);
-        et = groups_max(et);   // the tile's largest factor, the same in every lane
         const bool up = mt > m + kRowsLazy;   // as in attn_rows_mfma_kernel
         const float mn = up ? mt : m;
-        const float En = fmaxf(E, et);
-        if (__ballot(up || En != E)) {
-            const float alpha = !up ? 1.0f : m == -INFINITY ? 0.0f : expf(m - mn);
-            lsum *= alpha;
-            const float beta = alpha * (E / En);   // (E / En: powers of two)
-#pragma unroll
-            for (int b = 0; b < 16; b++) o[b] *= beta;
-        }
-        float p[8], ps = 0.0f;
+        float p[8], ps = 0.0f, T = 0.0f;      // weights, then times the V factors; their largest
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             p[e] = exp_le(val[e] ? sv[e] - mn : -200.0f);   // (e^-200 is 0)
             ps += p[e];
+            p[e] *= v4[e >> 2][e & 3];
+            T = fmaxf(T, p[e]);
+        }
+        T = groups_max(T);   // the same for both halves of the head
+        // E follows the row's largest product: up past 64 times it, and down with
+        // what is held when the running maximum moves
+        const float alpha = !up ? 1.0f : m == -INFINITY ? 0.0f : expf(m - mn);
+        const float Ea = E * alpha;
+        const float En = up || T > 64.0f * E ? fmaxf(__uint_as_float(__float_as_uint(fmaxf(Ea, T)) & 0x7f800000u), field_to_scale(6)) : E;
+        const int ef = (int)(__float_as_uint(En) >> 23);
+        if (__ballot(up || En != E)) {
+            lsum *= alpha;
+            const float beta = Ea * field_to_scale(254 - ef);   // alpha E / En
+#pragma unroll
+            for (int b = 0; b < 16; b++) o[b] *= beta;
         }
         lsum += ps;
         m = mn;
         E = En;
         ah8_t Ph, Pl;
-        const float u16 = field_to_scale(258 - (int)(__float_as_uint(E) >> 23));   // 16 / E
+        const float u16 = field_to_scale(258 - ef);   // 16 / E: weights below 2^11
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) {   // <= 16 e^kRowsLazy
+        for (int e = 0; e < 8; e += 2) {
             ah2_t h, l;
-            split2(p[e], p[e + 1], v4[e >> 2] * u16, h, l);
+            split2(p[e], p[e + 1], u16, h, l);
             Ph[e] = h[0];
             Ph[e + 1] = h[1];
             Pl[e] = l[0];

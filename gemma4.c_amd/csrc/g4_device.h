@@ -185,11 +185,12 @@ __device__ inline unsigned long long block_max_u64(unsigned long long k, unsigne
 
 typedef float f2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 h2v_t __attribute__((ext_vector_type(2)));
-// x sf and y sf as fp16 hi + lo (round to nearest; x sf - hi is exact)
-__device__ __forceinline__ void split2(float x, float y, float sf, h2v_t& hi, h2v_t& lo) {
-    hi = __builtin_convertvector((f2_t{x * sf, y * sf}), h2v_t);
-    lo = __builtin_convertvector((f2_t{__builtin_fmaf(x, sf, -(float)hi[0]), __builtin_fmaf(y, sf, -(float)hi[1])}), h2v_t);
+// x sx and y sy as fp16 hi + lo (round to nearest; x sx - hi is exact)
+__device__ __forceinline__ void split2(float x, float y, float sx, float sy, h2v_t& hi, h2v_t& lo) {
+    hi = __builtin_convertvector((f2_t{x * sx, y * sy}), h2v_t);
+    lo = __builtin_convertvector((f2_t{__builtin_fmaf(x, sx, -(float)hi[0]), __builtin_fmaf(y, sy, -(float)hi[1])}), h2v_t);
 }
+__device__ __forceinline__ void split2(float x, float y, float sf, h2v_t& hi, h2v_t& lo) { split2(x, y, sf, sf, hi, lo); }
 // max(|x|, |y|, m) in one instruction (fmaxf on loaded values is three)
 __device__ __forceinline__ float max3_abs(float x, float y, float m) {
     float r;

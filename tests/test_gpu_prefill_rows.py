@@ -397,3 +397,79 @@ def test_attn_decode_rows_512(lib, p0, m, G, window, ring, ks, vs):
             w = np.exp(s - s.max())
             want = (w / w.sum()) @ V64[t0:pos + 1, h // 4]
             assert np.abs(got[z, h] - want).max() <= 1e-5 * np.abs(want).max(), (z, h)
+
+
+def _rows512(lib, q, K, V, p0, G=1, window=0, ring=0, q8=False):
+    """g4_attn_decode_rows at head_dim 512 (8 query and 2 KV heads): K and V
+    hold positions 0 .. p0 + m - 1, slots and rows no query may read NaN"""
+    hd, n_heads, n_kv, m, T = 512, 8, 2, len(q), len(K)
+    kvd, slots = n_kv * hd, ring if ring else T
+    kc, vc = np.full((slots, kvd), np.nan, np.float32), np.full((slots, kvd), np.nan, np.float32)
+    for t in range(max(0, p0 - ring) if ring else 0, p0):
+        kc[t % slots], vc[t % slots] = K[t], V[t]
+    pad = np.full((2, kvd), np.nan, np.float32)
+    part = empty(lib, m * lib.L.g4_attn_part_bytes(n_heads, hd, G))
+    out = empty(lib, 4 * m * n_heads * hd)
+    q8b = empty(lib, m * lib.L.g4_q8K_row_stride(n_heads * hd)) if q8 else None
+    qd, kcd, vcd = dbuf(lib, q), dbuf(lib, kc), dbuf(lib, vc)
+    kchd, vchd = dbuf(lib, np.concatenate([K[p0:], pad])), dbuf(lib, np.concatenate([V[p0:], pad]))
+    lib.g4_attn_decode_rows(qd.ptr, kcd.ptr, vcd.ptr, kchd.ptr, vchd.ptr, kvd, ring, p0, m, window, n_heads, n_kv, hd,
+                            F(1.0), G, part.ptr, out.ptr, q8b.ptr if q8 else None)
+    return out.to_array(np.float32).reshape(m, n_heads, hd)
+
+
+def _attn64(q, K, V, t0, t1, h):
+    """head h (of 8 over 2 KV heads of 512) of query row q over positions t0 .. t1, in 64 bits"""
+    kv = slice(h // 4 * 512, h // 4 * 512 + 512)
+    s = K[t0:t1 + 1, kv].astype(np.float64) @ q[512 * h:512 * h + 512].astype(np.float64)
+    w = np.exp(s - s.max())
+    return (w / w.sum()) @ V[t0:t1 + 1, kv].astype(np.float64)
+
+
+@pytest.mark.parametrize("p0,m,G,window,ring", [(0, 24, 1, 0, 0), (70, 45, 3, 0, 0), (90, 40, 2, 20, 24)])
+@pytest.mark.parametrize("e", [12, 20, 40, 90])
+def test_attn_decode_rows_512_unseen_rows(lib, p0, m, G, window, ring, e):
+    """A key whose V, or K, is 2^e times larger does not touch the rows that may
+    not see it: those before it, and those whose window has passed it, are held
+    to the attention in 64 bits at 1e-5 of max|o|, as rows among keys of one size
+    are (test_attn_decode_rows_512)."""
+    hd, n_heads, n_kv = 512, 8, 2
+    rng = np.random.default_rng(p0 + m + e)
+    T = p0 + m
+    q = (rng.standard_normal((m, n_heads * hd)) * hd ** -0.5).astype(np.float32)
+    for big in (p0 + 5, p0 + 18, T - 1):
+        for which in "VK":
+            K, V = (rng.standard_normal((T, n_kv * hd)).astype(np.float32) for _ in "KV")
+            (V if which == "V" else K)[big] *= np.float32(2.0 ** e)
+            got = _rows512(lib, q, K, V, p0, G, window, ring)
+            for z in range(m):
+                t0 = max(0, p0 + z + 1 - window) if window else 0
+                if t0 <= big <= p0 + z:
+                    continue
+                for h in range(n_heads):
+                    want = _attn64(q[z], K, V, t0, p0 + z, h)
+                    assert np.abs(got[z, h] - want).max() <= 1e-5 * np.abs(want).max(), (which, big, z, h)
+
+
+@pytest.mark.parametrize("e", [20, 40, 60])
+def test_attn_decode_rows_512_light_keys(lib, e):
+    """A key whose V is 2^e times larger under a weight of about exp(-e - 12)
+    hardly adds to the output, and the keys that make it keep their precision
+    (1e-5 of max|o|), whether they come after it or before."""
+    hd, n_heads, n_kv, m = 512, 8, 2, 40
+    rng = np.random.default_rng(e)
+    q = (rng.standard_normal((m, n_heads * hd)) * 0.01).astype(np.float32)
+    q[:, ::hd] = 1.0                            # dim 0 of each head: the score of a key that holds only it
+    for at in (0, 7, 30):
+        K, V = (rng.standard_normal((m, n_kv * hd)).astype(np.float32) for _ in "KV")
+        K[:, ::hd] = 0.0
+        K[at] = 0.0
+        K[at, ::hd] = -(e + 12.0)
+        V[at] *= np.float32(2.0 ** e)
+        got = _rows512(lib, q, K, V, 0)
+        for z in range(m):
+            if z == at and at == 0:
+                continue                        # (its only key)
+            for h in range(n_heads):
+                want = _attn64(q[z], K, V, 0, z, h)
+                assert np.abs(got[z, h] - want).max() <= 1e-5 * np.abs(want).max(), (at, z, h)
