@@ -1658,6 +1658,11 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(2
 // the order in which a lane holds its weights.  Wave w stages keys 4w .. 4w + 3
 // whole, so a row's largest element is a reduction within the wave, and the
 // four rows' reductions share their steps.
+// Infinities and NaN: an infinite operand or an overflowing score leaves NaN in
+// the row (inf - inf in the split, exp_le); such rows, found by their results at
+// the end, are computed again by plain fp32 sums over the keys they see, one row
+// of a wave pair after the other.  That costs about 1.3 us for each row and key
+// (512 rows with one NaN among the first chunk's 512 V rows: 10.7 ms).
 // Two barriers a tile: V is split and staged between the score products, the
 // next tile's K between the output products, and each row's loads take the
 // registers of a row just staged (all 64 at once spilled: 470 us at the size
@@ -1670,7 +1675,8 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(2
 constexpr int kR5Keys = 32, kR5KRow = 2080;
 
 // e^x for x <= kRowsLazy, 0 below the smallest normal number: 2^(x log2 e) with
-// the product's rounding error put back to first order (within 2 ulp)
+// the product's rounding error put back to first order (within 2 ulp); NaN for
+// -inf and where x log2 e overflows
 __device__ __forceinline__ float exp_le(float x) {
     const float t = x * 1.44269504f;
     const float r = __builtin_fmaf(x, 1.92596303e-8f, __builtin_fmaf(x, 1.44269504f, -t));
@@ -1701,12 +1707,66 @@ __device__ __forceinline__ float rows_scale(const float (&m)[4], float (&sf)[4])
     return field_to_scale(254 - f);
 }
 
+// the partial of row zr over keys tb .. te in fp32 sums, one wave: dims 256 half ..
+// of the output, and from half 0 the (max, sum); four keys' loads at a time
+__device__ __forceinline__ void attn_row512_f32(const AttnArgs& a, int kvh, int zr, int tb, int te, int head, int half,
+                                                float* pp) {
+    constexpr int HD = 512;
+    const int lane = threadIdx.x & 63;
+    const float4* qv = reinterpret_cast<const float4*>(a.q + ((size_t)zr * a.n_heads + head) * HD);
+    const float4 q0 = qv[lane], q1 = qv[lane + 64];
+    float m = -INFINITY, l = 0.0f;
+    float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int t0 = tb; t0 <= te; t0 += 4) {
+        float s[4];
+        float4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int t = min(t0 + u, te);
+            const bool own = t >= a.p0;
+            const size_t off = (size_t)(own ? t - a.p0 : attn_slot(a, t)) * a.kv_stride + (size_t)kvh * HD;
+            const float4* kp = reinterpret_cast<const float4*>((own ? a.kchunk : a.kc) + off);
+            const float4 k0 = kp[lane], k1 = kp[lane + 64];
+            v[u] = reinterpret_cast<const float4*>((own ? a.vchunk : a.vc) + off)[64 * half + lane];
+            float d = k0.x * q0.x;
+            d = __builtin_fmaf(k0.y, q0.y, d);
+            d = __builtin_fmaf(k0.z, q0.z, d);
+            d = __builtin_fmaf(k0.w, q0.w, d);
+            d = __builtin_fmaf(k1.x, q1.x, d);
+            d = __builtin_fmaf(k1.y, q1.y, d);
+            d = __builtin_fmaf(k1.z, q1.z, d);
+            s[u] = a.scale * wave_sum(__builtin_fmaf(k1.w, q1.w, d));
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (t0 + u > te) break;
+            const float mn = fmaxf(m, s[u]);
+            const float al = m == mn ? 1.0f : m == -INFINITY ? 0.0f : expf(m - mn);
+            const float p = s[u] == -INFINITY ? 0.0f : expf(s[u] - mn);
+            l = l * al + p;
+            o.x = __builtin_fmaf(p, v[u].x, o.x * al);
+            o.y = __builtin_fmaf(p, v[u].y, o.y * al);
+            o.z = __builtin_fmaf(p, v[u].z, o.z * al);
+            o.w = __builtin_fmaf(p, v[u].w, o.w * al);
+            m = mn;
+        }
+    }
+    float2* out = reinterpret_cast<float2*>(pp + 256 * half) + 2 * lane;
+    out[0] = make_float2(o.x, o.y);
+    out[1] = make_float2(o.z, o.w);
+    if (lane == 0 && half == 0) {
+        pp[HD] = m;
+        pp[HD + 1] = l;
+    }
+}
+
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void attn_rows512_kernel(AttnArgs a) {
     constexpr int HD = 512;
     __shared__ __align__(16) uint8_t ks[kR5Keys * kR5KRow];
     __shared__ __align__(16) uint8_t vs[HD * 128];
     __shared__ __align__(16) float tsk[kR5Keys], tsv[kR5Keys];
     __shared__ __align__(16) f4_t ex[8][2][64];
+    __shared__ uint32_t badrows[8];
     const int c = blockIdx.x, kvh = blockIdx.y, rb = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, j = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave & 1;
@@ -1959,20 +2019,39 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
 
     lsum += __shfl_xor(lsum, 16, 64);
     lsum += __shfl_xor(lsum, 32, 64);
-    if (z < M) {
+    const float un = E * (1.0f / 16.0f);
+    float chk = lsum * 0.0f;   // NaN where a result of row j is not finite
+#pragma unroll
+    for (int b = 0; b < 16; b++) {
+        o[b] *= un;
+#pragma unroll
+        for (int r = 0; r < 4; r++) chk = __builtin_fmaf(o[b][r], 0.0f, chk);
+    }
+    const unsigned long long bad = __ballot(chk != 0.0f);
+    if (lane == 0) badrows[wave] = (uint32_t)(bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xffffu;
+    lds_sync();
+    // (the rows of either half: both write the same sums)
+    uint32_t again = __builtin_amdgcn_readfirstlane(badrows[wave & ~1] | badrows[wave | 1]);
+    float* const pz = a.part + ((size_t)head * a.G + c) * (HD + 2);
+    if (z < M && !(again >> j & 1)) {
         // o[b][r] is dim 256 half + 16 b + 4 g + r of row z
-        float* pp = a.part + (size_t)z * a.part_z + ((size_t)head * a.G + c) * (HD + 2);
-        const float un = E * (1.0f / 16.0f);
+        float* pp = pz + (size_t)z * a.part_z;
 #pragma unroll
         for (int b = 0; b < 16; b++) {
             float* q = pp + 256 * half + 16 * b + 4 * g;
-            *reinterpret_cast<float2*>(q) = make_float2(o[b][0] * un, o[b][1] * un);
-            *reinterpret_cast<float2*>(q + 2) = make_float2(o[b][2] * un, o[b][3] * un);
+            *reinterpret_cast<float2*>(q) = make_float2(o[b][0], o[b][1]);
+            *reinterpret_cast<float2*>(q + 2) = make_float2(o[b][2], o[b][3]);
         }
         if (g == 0 && half == 0) {
             pp[HD] = m;
             pp[HD + 1] = lsum;
         }
+    }
+    for (; again; again &= again - 1) {
+        const int zr = z0 + __builtin_ctz(again);
+        if (zr >= M) break;
+        attn_row512_f32(a, kvh, zr, max(cb, a.window > 0 ? a.p0 + zr + 1 - a.window : 0), min(a.p0 + zr, ce - 1), head, half,
+                        pz + (size_t)zr * a.part_z);
     }
 }
 

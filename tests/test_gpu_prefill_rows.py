@@ -473,3 +473,52 @@ def test_attn_decode_rows_512_light_keys(lib, e):
             for h in range(n_heads):
                 want = _attn64(q[z], K, V, 0, z, h)
                 assert np.abs(got[z, h] - want).max() <= 1e-5 * np.abs(want).max(), (at, z, h)
+
+
+def test_attn_decode_rows_512_not_finite(lib):
+    """Infinities, NaN and scores beyond the fp32 range at head_dim 512, by the
+    attention in 64 bits of what a row sees: a key whose score is -inf (one
+    infinity in K, or a product that overflows) has no weight; an infinite or
+    NaN element of V appears in its dimension and in no other, and in no row
+    that may not see the key; a NaN or infinite query leaves the other heads and
+    rows their bits.  At 1e-5 of the largest finite output, the bound of
+    test_attn_decode_rows_512."""
+    hd, n_heads, n_kv, p0, m = 512, 8, 2, 21, 40
+    rng = np.random.default_rng(8)
+    T = p0 + m
+    K, V = (rng.standard_normal((T, n_kv * hd)).astype(np.float32) for _ in "KV")
+    q = (rng.standard_normal((m, n_heads * hd)) * hd ** -0.5).astype(np.float32)
+    q[:, 9::hd] = rng.uniform(0.2, 3.0, (m, n_heads))
+    K[:, 9::hd] = 0.0
+
+    def check(got, drop, V):
+        for z in range(m):
+            seen = [t for t in range(p0 + z + 1) if t not in drop]
+            for h in range(n_heads):
+                fin = np.where(np.isfinite(V), V, 0.0)
+                want = _attn64(q[z], K[seen], fin[seen], 0, len(seen), h)
+                odd = V[seen, h // 4 * hd:h // 4 * hd + hd]
+                odd = np.where(np.isfinite(odd), 0.0, odd).sum(0)     # (weights are positive)
+                at = odd == 0
+                assert np.array_equal(got[z, h][~at], odd[~at].astype(np.float32), equal_nan=True), (z, h)
+                assert np.abs(got[z, h] - want)[at].max() <= 1e-5 * np.abs(want).max(), (z, h)
+
+    for G in (1, 4):
+        for at in (p0 + 3, p0 + 30, 11):
+            for k in (-np.inf, -3e38, -1e38):      # scores: -inf; -9e38 (overflows) .. -6e37; -3e38 .. -2e37
+                K2 = K.copy()
+                K2[at, 9::hd] = k
+                check(_rows512(lib, q, K2, V, p0, G), {at}, V)
+        K2 = K.copy()
+        K2[8:T, 9::hd] = -np.inf                   # chunks in which no key counts
+        check(_rows512(lib, q, K2, V, p0, G), set(range(8, T)), V)
+        for at in (p0 + 3, p0 + 30, 11):
+            V2 = V.copy()
+            V2[at, [3, 300, 515, 5]] = np.inf, -np.inf, np.inf, np.nan
+            check(_rows512(lib, q, K, V2, p0, G), set(), V2)
+        q2 = q.copy()
+        q2[7, 40], q2[20, 600], q2[33, 1100] = np.nan, np.inf, -np.inf
+        got, clean = _rows512(lib, q2, K, V, p0, G), _rows512(lib, q, K, V, p0, G)
+        for z, h in ((z, h) for z in range(m) for h in range(n_heads)):
+            if (z, h) not in ((7, 0), (20, 1), (33, 2)):
+                assert same_bits(got[z, h], clean[z, h]), (z, h)
