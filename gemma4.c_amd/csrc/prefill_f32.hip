@@ -30,6 +30,34 @@ namespace {
 
 typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
 
+// thread t of nt's part of the fp32 dot of a weight row and x (four elements in
+// nt * 4; nblk: Q6_K blocks of the matrix)
+template <bool BF>
+__device__ __forceinline__ float row_dot(const void* w, size_t nblk, const float* x, int n, size_t row, int t, int nt) {
+    f4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+    for (size_t k = 4 * (size_t)t; k < (size_t)n; k += 4 * (size_t)nt) {
+        const float4 xv = *reinterpret_cast<const float4*>(x + k);
+        float wv[4];
+        if (BF) {
+            const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(w) + row * n + k);
+            wv[0] = __uint_as_float(u.x << 16);
+            wv[1] = __uint_as_float(u.x & 0xffff0000u);
+            wv[2] = __uint_as_float(u.y << 16);
+            wv[3] = __uint_as_float(u.y & 0xffff0000u);
+        } else {
+            const size_t blk = row * ((size_t)n >> 8) + (k >> 8);
+#pragma unroll
+            for (int e = 0; e < 4; e++) wv[e] = dequant_elem(static_cast<const uint8_t*>(w), 14, nblk, blk, (int)(k & 255) + e);
+        }
+        s[0] = __builtin_fmaf(wv[0], xv.x, s[0]);
+        s[1] = __builtin_fmaf(wv[1], xv.y, s[1]);
+        s[2] = __builtin_fmaf(wv[2], xv.z, s[2]);
+        s[3] = __builtin_fmaf(wv[3], xv.w, s[3]);
+    }
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
 // the sum over the four waves' partial tiles and the store.  Weights are the
 // A operand: lane (g, i) holds weight rows 4g + v of 16-row group rt and token
 // i of 16-token group nt.  T: 16x16 tiles per wave; red_tiles(T) of them
@@ -494,6 +522,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     });
 }
 
+// Rows of 2^24 elements and more, where a tile's rows leave the 32-bit offsets of
+// the kernels above (Q6_K: sixteen rows of 5.7e8): a workgroup per output, every
+// address in 64 bits.
+template <bool BF>
+__global__ __launch_bounds__(256) void mm_batch_long_kernel(const void* w, const float* __restrict__ x, float* __restrict__ out,
+                                                            int n, int d) {
+    __shared__ float red[16];
+    const size_t row = blockIdx.x, tok = blockIdx.y;
+    const float s = block_sum(row_dot<BF>(w, (size_t)d * (n >> 8), x + tok * n, n, row, threadIdx.x, 256), red);
+    if (threadIdx.x == 0) out[tok * d + row] = s;
+}
+
 // Tile shapes.  The table holds the times in us of one workgroup on a CU and of
 // two that share it, with every CU taken (MI355X, 10240 columns, a sweep of all
 // shapes over 2..512 tokens); a launch runs in rounds of two a CU and the
@@ -567,17 +607,12 @@ extern "C" int g4_mm_batch_bf16_f32(float* o, const float* x, const void* w, int
 }
 
 int g4_mm_batch_f32(float* o, const float* x, const void* w, int n, int d, int m, int type) {
-    if (n < 1 << 24) {
-        const Tile& t = type == G4_BF16 ? pick_tile(kTilesBf16, d, m) : pick_tile(kTilesQ6, d, m);
-        t.launch(w, x, o, n, d, m);
-    } else {
-        // a tile's rows must lie within 32-bit offsets: one token (and bf16 row) a launch
-        for (int t = 0; t < m; t++)
-            for (int r = 0; r < (type == G4_BF16 ? d : 1); r++) {
-                const float* xt = x + (size_t)t * n;
-                if (type == G4_BF16) launch_bf16<1, 1>((const uint16_t*)w + (size_t)r * n, xt, o + (size_t)t * d + r, n, 1, 1);
-                else launch_q6<1, 1, 4>(w, xt, o + (size_t)t * d, n, d, 1);
-            }
+    if (n >= 1 << 24) {
+        if (type == G4_BF16) hipLaunchKernelGGL(mm_batch_long_kernel<true>, dim3(d, m), dim3(256), 0, g4_stream(), w, x, o, n, d);
+        else hipLaunchKernelGGL(mm_batch_long_kernel<false>, dim3(d, m), dim3(256), 0, g4_stream(), w, x, o, n, d);
+        return g4_check_launch("mm_batch_long_kernel");
     }
+    const Tile& t = type == G4_BF16 ? pick_tile(kTilesBf16, d, m) : pick_tile(kTilesQ6, d, m);
+    t.launch(w, x, o, n, d, m);
     return g4_check_launch(type == G4_BF16 ? "mm_batch_bf16_kernel" : "mm_batch_q6_kernel");
 }

@@ -493,6 +493,45 @@ def test_mm_batch_f32_not_finite(lib, qtype):
             assert np.array_equal(got[t].view(np.uint32), base[t].view(np.uint32)), t
 
 
+@pytest.mark.parametrize("qtype", [14, 30])
+def test_mm_batch_f32_long_rows(lib, qtype):
+    """Rows of 2^24 elements: within 1e-5 of sum |w x| of the exact product."""
+    from g4 import DBuf, upload_quant
+    rng = np.random.default_rng(2 + qtype)
+    n, d, m = 1 << 24, 3, 2
+    raw = synth.rand_bf16(rng, d, n) if qtype == 30 else synth.rand_q6K(rng, d, n)
+    w = DBuf.from_array(lib, raw) if qtype == 30 else upload_quant(lib, raw, 14, n, d)
+    x = rng.standard_normal((m, n), dtype=np.float32)
+    xd, out = DBuf.from_array(lib, x), DBuf(lib, 4 * m * d)
+    lib.g4_mm_batch(out.ptr, xd.ptr, w.ptr, n, d, m, qtype, None)
+    got = out.to_array(np.float32).reshape(m, d)
+    for r in range(d):
+        row = raw.reshape(d, -1)[r]
+        W = ((row.astype(np.uint32) << 16).view(np.float32).astype(np.float64) if qtype == 30
+             else kq.dequant_f64(row.reshape(-1, 210), 14).reshape(n))
+        for t in range(m):
+            assert abs(got[t, r] - W @ x[t]) <= TOL * (np.abs(W) @ np.abs(x[t])), (t, r)
+
+
+def test_mm_batch_f32_row_offsets_beyond_4_gib(lib):
+    """Sixteen Q6_K rows whose last begins more than 2^32 bytes of codes after the
+    first: every row its own weights.  All weights are zero but those of each
+    row's first and last block, 1 and r % 15 + 1 times the scale; x is constant."""
+    from g4 import DBuf
+    d, nb = 16, 2236968                               # 15 rows * 128 nb = 2^32 + 11 KiB
+    nblk, n = d * nb, 256 * nb
+    w, x, out = DBuf(lib, 210 * nblk), DBuf(lib, 4 * n), DBuf(lib, 4 * d)
+    for at, size, byte in ((0, 128, 0), (128, 64, 0xAA), (192, 16, 1), (208, 2, 0x3c)):   # ql, qh (code 32), sc, d
+        lib.check(lib.L.g4_memset(w.ptr + at * nblk, byte, size * nblk))
+    lib.check(lib.L.g4_memset(x.ptr, 0x3f, 4 * n))
+    for r in range(d):
+        w.write(np.full(128, 0x11, np.uint8), 128 * r * nb)
+        w.write(np.full(128, 0x11 * (r % 15 + 1), np.uint8), 128 * (r * nb + nb - 1))
+    lib.g4_mm_batch(out.ptr, x.ptr, w.ptr, n, d, 1, 14, None)
+    unit = 256 * float(np.uint32(0x3f3f3f3f).view(np.float32)) * float(np.uint16(0x3c3c).view(np.float16))
+    assert np.allclose(out.to_array(np.float32), unit * (2 + np.arange(d) % 15), rtol=1e-5)
+
+
 def test_mm_batch_bf16_f32(lib, orc):
     """The prompt path's bf16 GEMM: within 1e-5 of sum |w x| of mm_bf16
     (main.c:1529-1537), each token's bits its own."""
