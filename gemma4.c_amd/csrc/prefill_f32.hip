@@ -12,7 +12,10 @@
 // Wh + Wl as in mm_batch_q6s_kernel; three v_mfma_f32_16x16x32_f16, then one
 // multiplication by the token's scale and one FMA with the block's d.
 // Outputs that are not finite are computed again by plain fp32 dots, so
-// infinities and NaN in either operand behave as in the fp32 product.
+// infinities and NaN in either operand behave as in the fp32 product.  A wave
+// takes one dot after the other (Q6_K 2560 x 10240 over 512 tokens: 0.14 ms, with
+// one infinite token 0.9, all of them 12; bf16 10752 x 2560 0.13, 0.8, 19; with a
+// thread to a dot one token took 42 and 10 ms).
 //
 // Work split.  The four waves of a workgroup share one output tile and split
 // K: wave w takes the Q6_K blocks b = w (mod 4), or of every 256 bf16
@@ -35,7 +38,7 @@ typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
 template <bool BF>
 __device__ __forceinline__ float row_dot(const void* w, size_t nblk, const float* x, int n, size_t row, int t, int nt) {
     f4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 2
+#pragma unroll 4
     for (size_t k = 4 * (size_t)t; k < (size_t)n; k += 4 * (size_t)nt) {
         const float4 xv = *reinterpret_cast<const float4*>(x + k);
         float wv[4];
@@ -46,9 +49,18 @@ __device__ __forceinline__ float row_dot(const void* w, size_t nblk, const float
             wv[2] = __uint_as_float(u.y << 16);
             wv[3] = __uint_as_float(u.y & 0xffff0000u);
         } else {
+            // as dequant_elem, whose bytes for four elements in a row are a word each
             const size_t blk = row * ((size_t)n >> 8) + (k >> 8);
+            const Q6KPlanes P = q6k_planes(nblk);
+            const uint8_t* wb = static_cast<const uint8_t*>(w);
+            const int e0 = (int)(k & 255), h = e0 >> 7, kk = (e0 & 127) >> 5, l = e0 & 31;
+            const uint32_t ql = *reinterpret_cast<const uint32_t*>(wb + P.ql + blk * 128 + 64 * h + 16 * (l >> 3) + (l & 7) + 8 * (kk & 1));
+            const uint32_t qh = *reinterpret_cast<const uint32_t*>(wb + P.qh + blk * 64 + 32 * h + l);
+            const float sc = (float)(int8_t)wb[P.sc + blk * 16 + 8 * h + (l >> 4) + 2 * kk];
+            const float ds = hbits_to_f32(*reinterpret_cast<const uint16_t*>(wb + P.d + blk * 2)) * sc;
+            const uint32_t q = ((ql >> (4 * (kk >> 1))) & 0x0f0f0f0fu) | (((qh >> (2 * kk)) & 0x03030303u) << 4);
 #pragma unroll
-            for (int e = 0; e < 4; e++) wv[e] = dequant_elem(static_cast<const uint8_t*>(w), 14, nblk, blk, (int)(k & 255) + e);
+            for (int e = 0; e < 4; e++) wv[e] = ds * (float)((int)byte_of(q, e) - 32);
         }
         s[0] = __builtin_fmaf(wv[0], xv.x, s[0]);
         s[1] = __builtin_fmaf(wv[1], xv.y, s[1]);
@@ -64,9 +76,9 @@ __device__ __forceinline__ float row_dot(const void* w, size_t nblk, const float
 // pass through LDS at a time.
 constexpr int red_tiles(int t) { return t < 10 ? t : 10; }
 
-template <int NT, int RT, class Slow>
+template <int NT, int RT, class Dot>
 __device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, int part, float* __restrict__ out, int row0,
-                                             int tok0, int d, int m, bool vec, Slow slow) {
+                                             int tok0, int d, int m, bool vec, Dot part_dot) {
     constexpr int T = NT * RT, R = red_tiles(T);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -76,18 +88,22 @@ __device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, int
         for (int t = t0; t < t0 + R; t++)
             if (t < T) red[(part * R + (t - t0)) * 64 + lane] = acc[t / NT][t % NT];
         __syncthreads();
+        auto sums = [&](int u, float (&v)[4]) {   // tile t0 + u
+            const f4_t* r = red + u * 64 + lane;
+            const f4_t a = r[0], b = r[R * 64], c = r[2 * R * 64], e = r[3 * R * 64];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = (a[k] + b[k]) + (c[k] + e[k]);
+        };
+        uint32_t again = 0;   // the wave's tiles with an output that is not finite
 #pragma unroll
         for (int t = t0; t < t0 + R; t++) {
             if (t >= T || (t & 3) != wave) continue;
-            const f4_t* r = red + (t - t0) * 64 + lane;
-            const f4_t a = r[0], b = r[R * 64], c = r[2 * R * 64], e = r[3 * R * 64];
-            const int row = row0 + 16 * (t / NT) + 4 * g, tok = tok0 + 16 * (t % NT) + i;
-            float v[4];
+            float v[4], chk = 0.0f;
+            sums(t - t0, v);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                v[k] = (a[k] + b[k]) + (c[k] + e[k]);
-                if (tok < m && row + k < d && !(fabsf(v[k]) <= 3.402823466e38f)) v[k] = slow(tok, row + k);
-            }
+            for (int k = 0; k < 4; k++) chk = __builtin_fmaf(v[k], 0.0f, chk);
+            if (__ballot(chk != 0.0f)) again |= 1u << (t - t0);
+            const int row = row0 + 16 * (t / NT) + 4 * g, tok = tok0 + 16 * (t % NT) + i;
             if (tok >= m) continue;
             float* o = out + (size_t)tok * d + row;
             if (vec && row + 3 < d) {
@@ -96,6 +112,21 @@ __device__ __forceinline__ void reduce_store(f4_t (&acc)[RT][NT], f4_t* red, int
 #pragma unroll
                 for (int k = 0; k < 4; k++)
                     if (row + k < d) o[k] = v[k];
+            }
+        }
+        for (; again; again &= again - 1) {
+            const int u = __builtin_ctz(again), t = t0 + u;
+            const int row = row0 + 16 * (t / NT) + 4 * g, tok = tok0 + 16 * (t % NT) + i;
+            float v[4];
+            sums(u, v);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                unsigned long long todo = __ballot(tok < m && row + k < d && !(fabsf(v[k]) <= 3.402823466e38f));
+                for (; todo; todo &= todo - 1) {
+                    const int l = __builtin_ctzll(todo), tl = __builtin_amdgcn_readlane(tok, l), rl = __builtin_amdgcn_readlane(row, l) + k;
+                    const float s = wave_sum(part_dot(tl, rl));
+                    if (lane == l) out[(size_t)tl * d + rl] = s;
+                }
             }
         }
     }
@@ -207,10 +238,7 @@ __global__ __launch_bounds__(256) void mm_batch_bf16_kernel(const uint16_t* __re
     __syncthreads();
     f4_t* red = reinterpret_cast<f4_t*>(lds);
     reduce_store<NT, RT>(acc, red, wave, out, row0, tok0, d, m, vec, [&](int tok, int row) {
-        float sum = 0.0f;
-        for (int k = 0; k < n; k++)
-            sum = __builtin_fmaf(__uint_as_float((uint32_t)w[(size_t)row * n + k] << 16), x[(size_t)tok * n + k], sum);
-        return sum;
+        return row_dot<true>(w, 0, x + (size_t)tok * n, n, (size_t)row, lane, 64);
     });
 }
 
@@ -515,16 +543,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     __syncthreads();
     f4_t* red = reinterpret_cast<f4_t*>(lds);
     reduce_store<NT, RT>(acc, red, part, out, row0, tok0, d, m, vec, [&](int tok, int row) {
-        float sum = 0.0f;
-        for (int k = 0; k < n; k++)
-            sum = __builtin_fmaf(dequant_elem(w, 14, nblk, (size_t)row * nb + (k >> 8), k & 255), x[(size_t)tok * n + k], sum);
-        return sum;
+        return row_dot<false>(w, nblk, x + (size_t)tok * n, n, (size_t)row, lane, 64);
     });
 }
 
 // Rows of 2^24 elements and more, where a tile's rows leave the 32-bit offsets of
 // the kernels above (Q6_K: sixteen rows of 5.7e8): a workgroup per output, every
-// address in 64 bits.
+// address in 64 bits, bound by the loads that a workgroup keeps in flight.  16 rows
+// of 2^24, one / eight tokens: Q6_K 8.9 / 8.8 ms (28 / 224 in a launch a token),
+// bf16 7.4 / 7.1 (792 / 6490 in a launch an output).
 template <bool BF>
 __global__ __launch_bounds__(256) void mm_batch_long_kernel(const void* w, const float* __restrict__ x, float* __restrict__ out,
                                                             int n, int d) {

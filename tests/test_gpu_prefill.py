@@ -493,6 +493,35 @@ def test_mm_batch_f32_not_finite(lib, qtype):
             assert np.array_equal(got[t].view(np.uint32), base[t].view(np.uint32)), t
 
 
+@pytest.mark.parametrize("qtype,d,m", [(14, 10240, 300), (14, 2563, 64), (30, 10752, 512), (30, 4001, 80)])
+def test_mm_batch_f32_not_finite_large_tiles(lib, qtype, d, m):
+    """Outputs that are computed again in tiles of several LDS rounds: infinite
+    tokens in different rows and columns of a tile, among them the last; every
+    other token keeps its bits."""
+    from g4 import DBuf, upload_quant
+    rng = np.random.default_rng(d + m)
+    n = 256
+    raw = synth.rand_bf16(rng, d, n) if qtype == 30 else synth.rand_q6K(rng, d, n)
+    w = DBuf.from_array(lib, raw) if qtype == 30 else upload_quant(lib, raw, 14, n, d)
+    W = (raw.astype(np.uint32) << 16).view(np.float32) if qtype == 30 else kq.dequant_f64(raw.reshape(-1, 210), 14).astype(np.float32)
+    x = _acts(rng, m, n)
+    clean = DBuf.from_array(lib, x)
+    at = {1: np.inf, 18: -np.inf, 37: np.inf, m - 1: np.nan}
+    for t, v in at.items():
+        x[t, 3 * t % n] = v
+    xd, out, out2 = DBuf.from_array(lib, x), DBuf(lib, 4 * m * d), DBuf(lib, 4 * m * d)
+    lib.g4_mm_batch(out.ptr, xd.ptr, w.ptr, n, d, m, qtype, None)
+    lib.g4_mm_batch(out2.ptr, clean.ptr, w.ptr, n, d, m, qtype, None)
+    got, base = out.to_array(np.float32).reshape(m, d), out2.to_array(np.float32).reshape(m, d)
+    for t in range(m):
+        if t in at:
+            with np.errstate(invalid="ignore"):
+                want = W.reshape(d, n)[:, 3 * t % n] * np.float32(at[t])     # (the finite terms do not matter)
+            assert np.array_equal(got[t], want, equal_nan=True), t
+        else:
+            assert np.array_equal(got[t].view(np.uint32), base[t].view(np.uint32)), t
+
+
 @pytest.mark.parametrize("qtype", [14, 30])
 def test_mm_batch_f32_long_rows(lib, qtype):
     """Rows of 2^24 elements: within 1e-5 of sum |w x| of the exact product."""
