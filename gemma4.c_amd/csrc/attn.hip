@@ -2102,17 +2102,16 @@ void launch_merge(const AttnArgs& a, const dim3& grid) {
     else hipLaunchKernelGGL((attn_merge_kernel<HD, 128>), grid, dim3(256), 0, g4_stream(), a);
 }
 
-// head_dim 512 over query rows: attn_rows512_kernel (us, launch and merge,
-// against attn_rows_mfma_kernel<512>: 37 rows at position 0 21.7 / 26.6, 511 rows
-// 48.5 / 77, 512 rows at 1536 165 / 329, at 7680 360 / 872, 4 rows at 7000 63 /
-// 172; error against 64 bits 1.4e-7 .. 3.5e-7 / 1.7e-7 .. 5.0e-7).  The fp32 kernel
-// keeps the rows that are quantized on the spot (q8) within the first 1024
-// positions: an engine's prompt of that length goes through 8-bit codes in every
-// layer, where another order of sums moves some code by one and the model carries
-// it on, so it keeps the bits, and the tokens, it had.
-constexpr int kRowsQ8Keys = 1024;
-// up to 23 keys the 16-key tiles are faster (11 rows at 0: 19.2 / 18.0, 17: 21.6 /
-// 20.1, 24: 21.5 / 21.8)
+// head_dim 512 over query rows: attn_rows512_kernel where the result is wanted in
+// fp32 (us, launch and merge, against attn_rows_mfma_kernel<512>: 37 rows at
+// position 0 21.7 / 26.6, 511 rows 48.5 / 77, 512 rows at 1536 165 / 329, at 7680
+// 337 / 872, 4 rows at 7000 63 / 172; error against 64 bits 1.4e-7 .. 3.5e-7 / 1.7e-7
+// .. 5.0e-7).  Up to 23 keys the 16-key tiles are faster (11 rows at 0: 19.2 / 18.0,
+// 17: 21.6 / 20.1, 24: 21.5 / 21.8).  Rows that are quantized on the spot (q8: a
+// model's prompt) take the fp32 kernel at every length: their 8-bit codes go
+// through the layers that follow, where another order of sums moves some code by
+// one and the model carries it on, so a prompt keeps the bits, and the tokens, that
+// it has with fp32 products.
 constexpr int kRowsFewKeys = 23;
 
 int launch_attn(const AttnArgs& a) {
@@ -2128,7 +2127,7 @@ int launch_attn(const AttnArgs& a) {
             hipLaunchKernelGGL(attn_rows_h16_kernel<256>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
             launch_merge<256>(a, dim3(a.n_heads, 1, zq));
         } else {
-            if (a.p0 + a.qrows > (a.q8 ? kRowsQ8Keys : kRowsFewKeys)) hipLaunchKernelGGL(attn_rows512_kernel, rgrid, dim3(512), 0, g4_stream(), a);
+            if (!a.q8 && a.p0 + a.qrows > kRowsFewKeys) hipLaunchKernelGGL(attn_rows512_kernel, rgrid, dim3(512), 0, g4_stream(), a);
             else hipLaunchKernelGGL(attn_rows_mfma_kernel<512>, rgrid, dim3(64 * kRowsKVM), 0, g4_stream(), a);
             launch_merge<512>(a, dim3(a.n_heads, 2, zq));
         }

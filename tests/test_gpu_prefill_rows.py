@@ -212,6 +212,9 @@ ATTN_CASES = [
     (512, 8, 2, 0, 0, 300, 64, 3),         # full attention, flat cache
     (512, 2, 1, 0, 0, 0, 24, 1),           # the small test model's full layers
     (256, 8, 2, 512, 512, 0, 511, 4),      # the 511-token prompt of the decode workload
+    (512, 8, 2, 0, 0, 1000, 24, 16),       # global layers late in a prompt, around and past position 1024
+    (512, 8, 2, 0, 0, 1000, 25, 16),
+    (512, 8, 2, 0, 0, 1500, 40, 16),
 ]
 
 
@@ -522,3 +525,18 @@ def test_attn_decode_rows_512_not_finite(lib):
         for z, h in ((z, h) for z in range(m) for h in range(n_heads)):
             if (z, h) not in ((7, 0), (20, 1), (33, 2)):
                 assert same_bits(got[z, h], clean[z, h]), (z, h)
+
+
+@pytest.mark.parametrize("p0,m,more", [(1000, 24, 40), (3, 20, 60), (2000, 16, 17)])
+def test_attn_decode_rows_512_quantized_bits(lib, p0, m, more):
+    """Quantized rows at head_dim 512 (a prompt's global layers) have the same
+    bits whatever the rows after their 16-row block, up to position 1024 and
+    past it, and differ from the split form's by its rounding only."""
+    rng = np.random.default_rng(p0)
+    K, V = (rng.standard_normal((p0 + more, 1024)).astype(np.float32) for _ in "KV")
+    q = (rng.standard_normal((more, 4096)) * 512 ** -0.5).astype(np.float32)
+    few = _rows512(lib, q[:m], K[:p0 + m], V[:p0 + m], p0, 16, q8=True)
+    many = _rows512(lib, q, K, V, p0, 16, q8=True)
+    whole = m // 16 * 16
+    assert same_bits(few[:whole], many[:whole])
+    assert rel_err(_rows512(lib, q, K, V, p0, 16), many) <= 1e-5
