@@ -640,6 +640,8 @@ int g4_mm_batch_f32(float* o, const float* x, const void* w, int n, int d, int m
         return g4_check_launch("mm_batch_long_kernel");
     }
     const Tile& t = type == G4_BF16 ? pick_tile(kTilesBf16, d, m) : pick_tile(kTilesQ6, d, m);
-    t.launch(w, x, o, n, d, m);
+    // a grid holds fewer than 2^32 threads: outputs past 172 GB take several launches
+    const int gx = (d + 16 * t.rt - 1) / (16 * t.rt), step = max(1, (1 << 23) / gx) * 16 * t.nt;
+    for (int t0 = 0; t0 < m; t0 += step) t.launch(w, x + (size_t)t0 * n, o + (size_t)t0 * d, n, d, min(step, m - t0));
     return g4_check_launch(type == G4_BF16 ? "mm_batch_bf16_kernel" : "mm_batch_q6_kernel");
 }

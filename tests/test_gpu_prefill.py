@@ -561,6 +561,31 @@ def test_mm_batch_f32_row_offsets_beyond_4_gib(lib):
     assert np.allclose(out.to_array(np.float32), unit * (2 + np.arange(d) % 15), rtol=1e-5)
 
 
+def test_mm_batch_f32_many_workgroups(lib):
+    """An output of 171 GB: more than 2^24 workgroups of 256 threads, which one
+    launch cannot take.  Tokens at the start, in the middle and at the end have the
+    bits of a small batch."""
+    from g4 import DBuf, G4Error, upload_quant
+    n, d, m, rep = 256, 40964, 32705 * 32, 4960          # 513 x 32705 tiles of 80 rows x 32 tokens
+    try:
+        out = DBuf(lib, 4 * m * d)
+    except G4Error:
+        pytest.skip("171 GB of device memory are not free")
+    try:
+        rng = np.random.default_rng(1)
+        w = upload_quant(lib, synth.rand_q6K(rng, d, n), 14, n, d)
+        x = rng.standard_normal((rep, n)).astype(np.float32)
+        small, xd = DBuf(lib, 4 * 64 * d), DBuf.from_array(lib, np.tile(x, (m // rep, 1)))
+        lib.g4_mm_batch(out.ptr, xd.ptr, w.ptr, n, d, m, 14, None)
+        got = np.empty((64, d), np.float32)
+        for t in (0, 523232, m - 64):
+            lib.check(lib.L.g4_memcpy_d2h(P(got), out.ptr + 4 * t * d, got.nbytes))
+            lib.g4_mm_batch(small.ptr, xd.ptr + 4 * t * n, w.ptr, n, d, 64, 14, None)
+            assert np.array_equal(got.view(np.uint32).reshape(-1), small.to_array(np.uint32)), t
+    finally:
+        out.free()
+
+
 def test_mm_batch_bf16_f32(lib, orc):
     """The prompt path's bf16 GEMM: within 1e-5 of sum |w x| of mm_bf16
     (main.c:1529-1537), each token's bits its own."""
