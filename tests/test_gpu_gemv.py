@@ -395,11 +395,15 @@ def test_q6K_f32_gemv_row_lengths(lib, nb):
 
 
 @pytest.mark.parametrize("nb,d", [(4, 16384), (5, 32769), (6, 131073), (7, 16447), (8, 20001), (9, 16385), (10, 32700),
-                                  (11, 32769), (12, 16399)])
+                                  (11, 32769), (12, 16399), (4, 32700), (5, 32001), (7, 131075), (8, 131137), (9, 32701),
+                                  (11, 32703), (12, 32741)])
 def test_q6K_register_x_row_lengths(lib, orc, nb, d):
     """The register-x kernel at each row length, row counts that end inside a
     batch of 64: outputs to the GEMV bar, with the soft-cap (derivative <= 1) and
-    without, and the argmax key the first index of the largest output."""
+    without, and the argmax key the first index of the largest output.  (Without
+    soft-cap and argmax a launch takes the kernel where its last round is three
+    quarters full, and rows of 6 to 8 blocks from 131072 on: with 256 CUs at (6,
+    131073), (10, 32700) and the last seven sizes; the others take the K-slice kernel.)"""
     from g4 import DBuf, upload_quant
     n, cap = 256 * nb, 30.0
     rng = np.random.default_rng(nb + d)

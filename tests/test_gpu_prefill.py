@@ -408,8 +408,8 @@ def test_mm_batch_split_token_tiles(lib, d):
 @pytest.mark.parametrize("qtype", [14, 30])
 @pytest.mark.parametrize("n,d,m", [(2560, 512, 130), (256, 40, 5), (2560, 96, 1), (512, 10752, 33)])
 def test_mm_batch_f32_weights(lib, orc, qtype, n, d, m):
-    """The workspace-free g4_mm_batch for Q6_K and bf16 (the PLE projection):
-    fp32 matrix-core sums of the reference's dequantized weights, sampled
+    """The workspace-free g4_mm_batch for Q6_K and bf16 (the PLE projection's
+    shapes): sums of the reference's dequantized weights, sampled
     tokens within 1e-5 of sum |w x| of mm_quant_rows / mm_bf16
     (main.c:1539-1556, 1529-1537), shift-invariant bit for bit."""
     from g4 import DBuf, upload_quant
@@ -435,7 +435,8 @@ def test_mm_batch_f32_weights(lib, orc, qtype, n, d, m):
 def test_mm_batch_f32_tiles(lib, qtype, n, d):
     """Every tile shape of the Q6_K / bf16 GEMM on fp32 activations (batches of
     1 to 600 tokens, rows that end inside a tile, an output that is only
-    4-byte aligned): a token's bits are the same in each, and within 1e-6 of
+    4-byte aligned; with 256 CUs the bf16 tile of 32 tokens x 64 rows is taken
+    at 4099 rows and 200 tokens, the others at several of the sizes): a token's bits are the same in each, and within 1e-6 of
     sum |w x| of the exact product (24-bit products and sums: 2^-22 an element
     of the split, 2^-24 a sum, of which 1e-6 leaves a factor of three)."""
     from g4 import DBuf, upload_quant
@@ -451,7 +452,7 @@ def test_mm_batch_f32_tiles(lib, qtype, n, d):
     W64, X64 = W.reshape(d, n).astype(np.float64), x.astype(np.float64)
     want, mag = X64 @ W64.T, np.abs(X64) @ np.abs(W64).T
     ref = None
-    for m in (600, 1, 5, 16, 17, 37, 64, 130, 257):
+    for m in (600, 1, 5, 16, 17, 37, 64, 130, 200, 257):
         lib.g4_mm_batch(out.ptr + 4 * (m & 1), xd.ptr, w.ptr, n, d, m, qtype, None)
         got = out.to_array(np.float32)[(m & 1):(m & 1) + m * d].reshape(m, d)
         if ref is None:

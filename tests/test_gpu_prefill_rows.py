@@ -314,8 +314,8 @@ def test_residual_norm_rows(lib, n, narrow):
 
 @pytest.mark.parametrize("hd", [256, 512])
 def test_attn_decode_rows_peaked_small(lib, orc, hd):
-    """The prompt-chunk attention (hd 256: split-fp16 matrix cores; 512: fp32
-    ones) with small-magnitude queries (elements ~0.05, their fp16 low parts
+    """The prompt-chunk attention (split-fp16 matrix cores at both head sizes)
+    with small-magnitude queries (elements ~0.05, their fp16 low parts
     subnormal) against large keys, so that the softmax is peaked and most
     weights lie in 1e-3..1e-1 -- where a weight split without its factor 16
     would keep only 2^-15 of relative precision -- compared with the oracle
@@ -370,9 +370,9 @@ ROWS512_CASES = [
 def test_attn_decode_rows_512(lib, p0, m, G, window, ring, ks, vs):
     """head_dim 512 on split fp16 products against the attention in 64 bits:
     every element is held to 2^-22, so a score of |s| <= 6 is off by less than
-    2^-20 and the output by less than 1e-5 of max|o|.  Key rows differ in size by
-    factors up to 2^8, so that the per-row-group scales change between tiles;
-    rows no query may read hold NaN."""
+    2^-20 and the output by less than 1e-5 of max|o|.  V rows differ in size by factors
+    up to 2^7, so that every key has a scale of its own (larger ones, and of K, in
+    the tests below); rows no query may read hold NaN."""
     hd, n_heads, n_kv = 512, 8, 2
     rng = np.random.default_rng(p0 + m + G)
     kvd, T = n_kv * hd, p0 + m
