@@ -1413,6 +1413,14 @@ __device__ __forceinline__ float groups_max(float v) {
     const auto q = __builtin_amdgcn_permlane16_swap(w, w, false, false);
     return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
+// their sum, (v(j) + v(j + 16)) + (v(j + 32) + v(j + 48))
+__device__ __forceinline__ float groups_sum(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const uint32_t w = __float_as_uint(__uint_as_float(p[0]) + __uint_as_float(p[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
 __device__ __forceinline__ _Float16 split_hi(float v) { return (_Float16)v; }
 __device__ __forceinline__ _Float16 split_lo(float v, _Float16 h) { return (_Float16)(v - (float)h); }
 
@@ -1666,12 +1674,12 @@ __global__ __launch_bounds__(64 * kRowsKVM) __attribute__((amdgpu_waves_per_eu(2
 // Two barriers a tile: V is split and staged between the score products, the
 // next tile's K between the output products, and each row's loads take the
 // registers of a row just staged (all 64 at once spilled: 470 us at the size
-// below).  512 rows at positions 7680 .. 8191, 16 chunks: 872 us on the fp32
-// matrix cores; here 545 with the addresses behind branches (each load waited
-// for all before it), 465 without, 419 with operands read ahead of their
-// products, 360 with the splits between the products.  What is left is VALU
-// issue (half of the time) and the matrix cores (a quarter), which a wave
-// overlaps only in part.
+// below).  512 rows at positions 7680 .. 8191, 16 chunks, with the merge: 872 us on
+// the fp32 matrix cores; here 545 with the addresses behind branches (each load
+// waited for all before it), 465 without, 419 with operands read ahead of their
+// products, 360 with the splits between the products (377 on a slower card, 335 to
+// 345 in turn with other launches).  What is left is VALU issue (half of the time)
+// and the matrix cores (a quarter), which a wave overlaps only in part.
 constexpr int kR5Keys = 32, kR5KRow = 2080;
 
 // e^x for x <= kRowsLazy, 0 below the smallest normal number: 2^(x log2 e) with
@@ -1861,9 +1869,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
         for (int s = 0; s < 8; s++)
 #pragma unroll
             for (int t = 0; t < 8; t++) mx = fmaxf(mx, fabsf(qrow[32 * s + t]));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const int f = scale_field(mx);
+        const int f = scale_field(groups_max(mx));
         const float sf = field_to_scale(f);
         tsq = field_to_scale(254 - f);
 #pragma unroll
@@ -1975,11 +1981,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
 #pragma unroll
             for (int b = 0; b < 16; b++) o[b] *= beta;
         }
+        E = En;
         lsum += ps;
         m = mn;
-        E = En;
         ah8_t Ph, Pl;
-        const float u16 = field_to_scale(258 - ef);   // 16 / E: weights below 2^11
+        const float u16 = field_to_scale(258 - (int)(__float_as_uint(E) >> 23));   // 16 / E: weights below 2^11
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
             ah2_t h, l;
@@ -2017,32 +2023,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
         }
     }
 
-    lsum += __shfl_xor(lsum, 16, 64);
-    lsum += __shfl_xor(lsum, 32, 64);
+    lsum = groups_sum(lsum);
+    // the lane number anew: kept through the loop it would take a spill, whose reload waits here
+    int none = 0;
+    asm volatile("" : "+s"(none));
+    const int le = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none)), ge = le >> 4, je = le & 15, ze = z0 + je;
     const float un = E * (1.0f / 16.0f);
-    float chk = lsum * 0.0f;   // NaN where a result of row j is not finite
+    f4_t chk = {lsum * 0.0f, 0.0f, 0.0f, 0.0f};   // NaN where a result of row j is not finite
 #pragma unroll
     for (int b = 0; b < 16; b++) {
         o[b] *= un;
 #pragma unroll
-        for (int r = 0; r < 4; r++) chk = __builtin_fmaf(o[b][r], 0.0f, chk);
+        for (int r = 0; r < 4; r++) chk[r] = __builtin_fmaf(o[b][r], 0.0f, chk[r]);
     }
-    const unsigned long long bad = __ballot(chk != 0.0f);
-    if (lane == 0) badrows[wave] = (uint32_t)(bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xffffu;
+    const unsigned long long bad = __ballot((chk[0] + chk[1]) + (chk[2] + chk[3]) != 0.0f);
+    if (le == 0) badrows[wave] = (uint32_t)(bad | bad >> 16 | bad >> 32 | bad >> 48) & 0xffffu;
     lds_sync();
     // (the rows of either half: both write the same sums)
     uint32_t again = __builtin_amdgcn_readfirstlane(badrows[wave & ~1] | badrows[wave | 1]);
     float* const pz = a.part + ((size_t)head * a.G + c) * (HD + 2);
-    if (z < M && !(again >> j & 1)) {
-        // o[b][r] is dim 256 half + 16 b + 4 g + r of row z
-        float* pp = pz + (size_t)z * a.part_z;
+    if (ze < M && !(again >> je & 1)) {
+        // o[b][r] is dim 256 half + 16 b + 4 ge + r of row ze
+        float* pp = pz + (size_t)ze * a.part_z;
 #pragma unroll
         for (int b = 0; b < 16; b++) {
-            float* q = pp + 256 * half + 16 * b + 4 * g;
+            float* q = pp + 256 * half + 16 * b + 4 * ge;
             *reinterpret_cast<float2*>(q) = make_float2(o[b][0], o[b][1]);
             *reinterpret_cast<float2*>(q + 2) = make_float2(o[b][2], o[b][3]);
         }
-        if (g == 0 && half == 0) {
+        if (ge == 0 && half == 0) {
             pp[HD] = m;
             pp[HD + 1] = lsum;
         }
@@ -2104,14 +2113,14 @@ void launch_merge(const AttnArgs& a, const dim3& grid) {
 
 // head_dim 512 over query rows: attn_rows512_kernel where the result is wanted in
 // fp32 (us, launch and merge, against attn_rows_mfma_kernel<512>: 37 rows at
-// position 0 21.7 / 26.6, 511 rows 48.5 / 77, 512 rows at 1536 165 / 329, at 7680
-// 337 / 872, 4 rows at 7000 63 / 172; error against 64 bits 1.4e-7 .. 3.5e-7 / 1.7e-7
-// .. 5.0e-7).  Up to 23 keys the 16-key tiles are faster (11 rows at 0: 19.2 / 18.0,
-// 17: 21.6 / 20.1, 24: 21.5 / 21.8).  Rows that are quantized on the spot (q8: a
-// model's prompt) take the fp32 kernel at every length: their 8-bit codes go
-// through the layers that follow, where another order of sums moves some code by
-// one and the model carries it on, so a prompt keeps the bits, and the tokens, that
-// it has with fp32 products.
+// position 0 22.8 / 26.9, 511 rows 49 / 76, 512 rows at 1536 169 / 332, at 7680 360 to
+// 377 / 854 to 878, 4 rows at 7000 63 / 173; error against 64 bits 1.4e-7 .. 3.5e-7
+// / 1.7e-7 .. 5.0e-7).  Up to 23 keys the 16-key tiles are as fast or faster (24 rows
+// at 0: 22.1 / 21.8, 28: 22.1 / 23.5; 4 rows at 20 are at 16.1 / 20.6).
+// Rows that are quantized on the spot (q8: a model's prompt) take the fp32 kernel at
+// every length: their 8-bit codes go through the layers that follow, where another
+// order of sums moves some code by one and the model carries it on, so a prompt keeps
+// the bits, and the tokens, that it has with fp32 products.
 constexpr int kRowsFewKeys = 23;
 
 int launch_attn(const AttnArgs& a) {
