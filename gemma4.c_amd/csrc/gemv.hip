@@ -723,7 +723,7 @@ __global__ __launch_bounds__(64 * kPleNB) void ple_fused_kernel(const uint8_t* _
 }
 
 // ------------------------------------------------------------------------
-// Q4_K / Q5_K x Q8_K, streaming form (rows of 8, 10 or 16 blocks)
+// Q4_K / Q5_K x Q8_K, streaming form (rows of 2 to 10 or 16 blocks)
 // ------------------------------------------------------------------------
 // One wave per workgroup; an 8-lane group owns one row of one matrix and
 // runs all NB blocks of it in order, so no lane shuffles are needed between

@@ -514,8 +514,9 @@ __global__ __launch_bounds__(64 * NWV) void mm_batch_kq8w_kernel(const KqSegs sg
 }
 
 // Waves over K of mm_batch_kq8w_kernel, or 0 where mm_batch_kq8_kernel is faster:
-// while a CU has at most three workgroups of 32 rows x 32 tokens (five of the
-// eight-wave ones, two of which it holds at once), and more than one block.  us,
+// while a CU has at most three workgroups of 32 rows x 32 tokens (five for rows of
+// up to eight blocks, whose 2, 4 or 8 waves leave room for two and more at once; a
+// CU holds one of ten waves), and more than one block.  us,
 // here against there:
 //   10240 x 2560: 8 tokens (320 workgroups) 11.9 / 20.5, 37 (640) 17.3 / 21.1, 130
 //     (1600) 36.5 / 26.2

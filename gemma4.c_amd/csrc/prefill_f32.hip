@@ -8,7 +8,8 @@
 // v_mfma_f32_16x16x32_bf16 give the fp32 path's products exactly.  Q6_K: over
 // 64 elements of a token the activations are scaled by the power of two that
 // brings the largest into [2^14, 2^15) and split into two fp16 terms (within
-// 2^-22 of each element), the integer weight sc * (q - 32) exactly into
+// 2^-22 of an element or 2^-39 of the largest of the 64, whichever is more; the
+// product of both low terms, below 2^-22 of its term, is left out), the integer weight sc * (q - 32) exactly into
 // Wh + Wl as in mm_batch_q6s_kernel; three v_mfma_f32_16x16x32_f16, then one
 // multiplication by the token's scale and one FMA with the block's d.
 // Outputs that are not finite are computed again by plain fp32 dots, so

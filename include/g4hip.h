@@ -266,8 +266,10 @@ int g4_fold_gelu_mul_q8(const float *u, const void *q8, int n, const float *ple,
 /* m tokens through mm(o_t, x_t, w, n, d, type, q8, 0) (main.c:1669): Q4_K /
  * Q5_K quantize all rows into q8 (m * g4_q8K_row_stride(n) bytes) and take
  * g4_mm_batch_q8; Q6_K and BF16 with n a multiple of 256 and 16-byte aligned
- * x, w: one matrix-core GEMM on the fp32 activations (split into 16-bit terms;
- * the reference's dequantized weights, fp32 sums in another order; q8 unused);
+ * x, w: one matrix-core GEMM on the fp32 activations (bf16: split exactly;
+ * Q6_K: an activation within 2^-22 of its value or 2^-39 of the largest of its
+ * 64; the reference's dequantized weights, fp32 sums in another order; q8
+ * unused; outputs that are not finite are computed as fp32 dots, a wave each);
  * otherwise the per-token GEMV m times. */
 int g4_mm_batch(float *o, const float *x, const void *w, int n, int d, int m, int type, void *q8);
 /* g4_mm_batch of a bf16 matrix (n a multiple of 256; x, w 16-byte aligned) with
@@ -333,7 +335,11 @@ int g4_kv_store_rows(float *kc, float *vc, const float *kin, const float *vin, i
                      int kvd);
 /* the attention block (main.c:1909-1950) for m query rows at positions
  * p0..p0+m-1: the chunk's K/V in rows of kchunk/vchunk, earlier positions in
- * the cache (ring: window <= ring); part: m * g4_attn_part_bytes(n_heads, hd, G) */
+ * the cache (ring: window <= ring); part: m * g4_attn_part_bytes(n_heads, hd, G).
+ * Without q8 (fp32 outputs alone) head_dim 512 runs on split fp16 products: an
+ * element of a K or V row or of half a q row is within 2^-22 of its value or
+ * 2^-39 of that row's largest; rows with infinities or NaN among what they see
+ * are fp32 sums, about 1.3 us for each row and key */
 int g4_attn_decode_rows(const float *q, const float *kc, const float *vc, const float *kchunk, const float *vchunk,
                         int kv_stride, int ring, int p0, int m, int window, int n_heads, int n_kv, int hd,
                         float attn_scale, int G, float *part, float *out, void *q8);
