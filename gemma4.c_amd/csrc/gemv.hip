@@ -1260,7 +1260,7 @@ constexpr int kQ6SliceRows = 5;       // 512 workgroups at the FFN-down shape: t
 constexpr int kQ6SliceMaxNb = 64;
 constexpr int kQ6SliceIdleRows = 40000;
 
-template <int R>
+template <int R, bool WHOLE>
 __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(const uint8_t* __restrict__ w,
                                                                           const float* __restrict__ x,
                                                                           float* __restrict__ out, int nb, int d) {
@@ -1268,7 +1268,9 @@ __global__ __launch_bounds__(8 * kQ6SliceMaxNb) void gemv_q6k_kslice_kernel(cons
     const int tid = threadIdx.x, L = tid & 7, g = tid >> 3, h = L >> 2, u = L & 3;
     const int r0 = blockIdx.x * R;
     const Q6KPlanes P = q6k_planes((size_t)d * nb);
-    const int gb = min(g, nb - 1);   // (whole waves: groups past the row repeat its last block, unused)
+    // groups past the row repeat its last block, unused.  (WHOLE: rows that fill the
+    // waves have none; with the clamp a launch of 2560 rows of 40 blocks took 0.15 us more)
+    const int gb = WHOLE ? g : min(g, nb - 1);
     // x of this lane first (runs k = 0..3 of 8 elements at g*256 + 128h +
     // 32k + 8u), then every weight load of the R rows, all issued before
     // anything waits: the load counter retires in order, so the run sums
@@ -1726,8 +1728,10 @@ int launch_q6_f32(const void* w, const float* x, float* o, int nb, int d, float 
     // blocks 8.5 / 13.7 -> 4.8 / 7.6 us, 40000 of 15 33.9 -> 24.7).
     const int groups = (nb + 7) & ~7;
     if (!SOFTCAP && nb <= kQ6SliceMaxNb && (d <= kQ6SliceIdleRows || 3 * (groups - nb) < groups)) {
-        hipLaunchKernelGGL((gemv_q6k_kslice_kernel<kQ6SliceRows>), dim3((d + kQ6SliceRows - 1) / kQ6SliceRows),
-                           dim3(8 * groups), 0, g4_stream(), (const uint8_t*)w, x, o, nb, d);
+        const dim3 grid((d + kQ6SliceRows - 1) / kQ6SliceRows), block(8 * groups);
+        const uint8_t* wp = (const uint8_t*)w;
+        if (nb == groups) hipLaunchKernelGGL((gemv_q6k_kslice_kernel<kQ6SliceRows, true>), grid, block, 0, g4_stream(), wp, x, o, nb, d);
+        else hipLaunchKernelGGL((gemv_q6k_kslice_kernel<kQ6SliceRows, false>), grid, block, 0, g4_stream(), wp, x, o, nb, d);
         return g4_check_launch("gemv_q6k_kslice_kernel");
     }
     const int target = 2 * g4_num_cus();
