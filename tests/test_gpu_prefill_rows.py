@@ -478,7 +478,8 @@ def test_attn_decode_rows_512_light_keys(lib, e):
                 assert np.abs(got[z, h] - want).max() <= 1e-5 * np.abs(want).max(), (at, z, h)
 
 
-def test_attn_decode_rows_512_not_finite(lib):
+@pytest.mark.parametrize("window,ring", [(0, 0), (20, 24)])
+def test_attn_decode_rows_512_not_finite(lib, window, ring):
     """Infinities, NaN and scores beyond the fp32 range at head_dim 512, by the
     attention in 64 bits of what a row sees: a key whose score is -inf (one
     infinity in K, or a product that overflows) has no weight; an infinite or
@@ -496,7 +497,7 @@ def test_attn_decode_rows_512_not_finite(lib):
 
     def check(got, drop, V):
         for z in range(m):
-            seen = [t for t in range(p0 + z + 1) if t not in drop]
+            seen = [t for t in range(max(0, p0 + z + 1 - window) if window else 0, p0 + z + 1) if t not in drop]
             for h in range(n_heads):
                 fin = np.where(np.isfinite(V), V, 0.0)
                 want = _attn64(q[z], K[seen], fin[seen], 0, len(seen), h)
@@ -511,17 +512,18 @@ def test_attn_decode_rows_512_not_finite(lib):
             for k in (-np.inf, -3e38, -1e38):      # scores: -inf; -9e38 (overflows) .. -6e37; -3e38 .. -2e37
                 K2 = K.copy()
                 K2[at, 9::hd] = k
-                check(_rows512(lib, q, K2, V, p0, G), {at}, V)
+                check(_rows512(lib, q, K2, V, p0, G, window, ring), {at}, V)
         K2 = K.copy()
-        K2[8:T, 9::hd] = -np.inf                   # chunks in which no key counts
-        check(_rows512(lib, q, K2, V, p0, G), set(range(8, T)), V)
+        off = [t for t in range(8, T) if not window or t % 10]
+        K2[off, 9::hd] = -np.inf                   # (without a window: chunks in which no key counts)
+        check(_rows512(lib, q, K2, V, p0, G, window, ring), set(off), V)
         for at in (p0 + 3, p0 + 30, 11):
             V2 = V.copy()
             V2[at, [3, 300, 515, 5]] = np.inf, -np.inf, np.inf, np.nan
-            check(_rows512(lib, q, K, V2, p0, G), set(), V2)
+            check(_rows512(lib, q, K, V2, p0, G, window, ring), set(), V2)
         q2 = q.copy()
         q2[7, 40], q2[20, 600], q2[33, 1100] = np.nan, np.inf, -np.inf
-        got, clean = _rows512(lib, q2, K, V, p0, G), _rows512(lib, q, K, V, p0, G)
+        got, clean = _rows512(lib, q2, K, V, p0, G, window, ring), _rows512(lib, q, K, V, p0, G, window, ring)
         for z, h in ((z, h) for z in range(m) for h in range(n_heads)):
             if (z, h) not in ((7, 0), (20, 1), (33, 2)):
                 assert same_bits(got[z, h], clean[z, h]), (z, h)
